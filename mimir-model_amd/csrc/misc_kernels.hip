@@ -1,6 +1,5 @@
 // Smaller kernels of the path: the per-row refusal scan of a weight, block
-// decode (mim.Dequantize), the float32-activation product
-// (dequant_matmul.v1), and the Q8_0 x 8-bit block-32 GEMV.
+// decode (mim.Dequantize) and the Q8_0 x 8-bit block-32 GEMV.
 #include "f32path.hpp"
 #include "mimg_device.hpp"
 #include "mimg_kernels.hpp"
@@ -51,43 +50,6 @@ hipError_t launch_dequantize(uint32_t dt, const uint8_t* src, int64_t n, float* 
     case DT_Q4_K: hipLaunchKernelGGL(dequantize_kernel<DT_Q4_K>, grid, blk, 0, stream, src, n, dst); break;
     case DT_Q6_K: hipLaunchKernelGGL(dequantize_kernel<DT_Q6_K>, grid, blk, 0, stream, src, n, dst); break;
     case DT_Q8_0: hipLaunchKernelGGL(dequantize_kernel<DT_Q8_0>, grid, blk, 0, stream, src, n, dst); break;
-    default: return hipErrorInvalidValue;
-    }
-    return hipGetLastError();
-}
-
-// dequant_matmul.v1 (reference linearF32/linearCols, interp/fast.go:161-183):
-// one group of eight lanes per (weight row j, activation row i), the product
-// in the reference's float order (f32path.hpp), then s + bias[j].
-template <uint32_t DT>
-__global__ __launch_bounds__(256) void linear_f32_kernel(const uint8_t* __restrict__ W, int64_t rb,
-                                                         int64_t N, int64_t K,
-                                                         const float* __restrict__ x, int64_t rows,
-                                                         const float* __restrict__ bias,
-                                                         float* __restrict__ y) {
-    const int64_t pair = (int64_t)blockIdx.x * 32 + (threadIdx.x >> 3);
-    const int64_t pc = pair < N * rows ? pair : N * rows - 1;
-    const int64_t i = pc / N, j = pc - i * N;
-    float r = f32dot_g8<DT>(W + j * rb, x + i * K, K, rows <= 8);
-    if (bias) r += bias[j];
-    if ((threadIdx.x & 7) == 0 && pair < N * rows) y[i * N + j] = r;
-}
-
-hipError_t launch_linear_f32(const DevWeight& w, const float* x, int64_t rows, const float* bias,
-                             float* y, hipStream_t stream) {
-    if (rows <= 0 || w.n <= 0) return hipSuccess;
-    int64_t pairs = rows * w.n;
-    dim3 grid((unsigned)((pairs + 31) / 32)), blk(256);
-    switch (w.dt) {
-    case DT_Q4_K:
-        hipLaunchKernelGGL(linear_f32_kernel<DT_Q4_K>, grid, blk, 0, stream, w.data, w.row_bytes, w.n, w.k, x, rows, bias, y);
-        break;
-    case DT_Q6_K:
-        hipLaunchKernelGGL(linear_f32_kernel<DT_Q6_K>, grid, blk, 0, stream, w.data, w.row_bytes, w.n, w.k, x, rows, bias, y);
-        break;
-    case DT_Q8_0:
-        hipLaunchKernelGGL(linear_f32_kernel<DT_Q8_0>, grid, blk, 0, stream, w.data, w.row_bytes, w.n, w.k, x, rows, bias, y);
-        break;
     default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
