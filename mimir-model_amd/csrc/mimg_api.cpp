@@ -364,6 +364,11 @@ bool fused_q8_blocks(uint32_t dt, int block) {
 // (bit-identical to the GEMV) instead of the GEMV in chunks of eight rows.
 constexpr int64_t GEMM_MIN_ROWS = 16;
 
+// The same for blocks of 32, whose tiles keep the reference's lane order
+// (measured with the quantizer, 4096 x 4096 Q8_0: 27 us in tiles at 9..32
+// rows, 17.5 in the GEMV at 8, twice that at 9).
+constexpr int64_t GEMM_B32_MIN_ROWS = 9;
+
 // Every workgroup of a product reads all of x (the float32 path of refused
 // rows included) while others write y: y[i] must not overlap x.
 static int check_outputs(const float* x, int64_t rows, int64_t K, const int64_t* N, float* const* y, int count) {
@@ -385,8 +390,8 @@ constexpr int64_t MFMA_MIN_ROWS = 4;
 // quantized into `a`; block-256 weights of one dtype share a launch per
 // chunk of 8 rows. Every path keeps each row's result independent of the
 // other rows of the call: block 256 from GEMM_MIN_ROWS on the MFMA GEMM
-// (bit-identical to the GEMV), blocks of 32 always the GEMV in the
-// reference's lane order.
+// and blocks of 32 from GEMM_B32_MIN_ROWS on their own (Q8_0), each
+// bit-identical to its GEMV, which takes the rest in chunks of eight.
 int matmul_quantized(const Weight* const* w, int count, const float* x, int64_t rows, const float* const* bias,
                      int block, float* const* y, const ActPtrs& a, hipStream_t s) {
     const int64_t K = w[0]->dw.k, R32 = K / 32, R16 = K / 16;
@@ -401,6 +406,18 @@ int matmul_quantized(const Weight* const* w, int count, const float* x, int64_t 
             return MIMG_OK;
         }
     }
+    bool tiled[3] = {false, false, false};
+    if (block == 32 && rows >= GEMM_B32_MIN_ROWS) {
+        int left = count;
+        for (int i = 0; i < count; i++) {
+            if (w[i]->dw.dt != DT_Q8_0) continue;
+            hipError_t e = launch_gemm_q8_0_ref(w[i]->dw, a, rows, rows, x, bias ? bias[i] : nullptr, y[i], s);
+            if (e != hipSuccess) return fail(MIMG_ERR_HIP, "GEMM launch: %s", hipGetErrorString(e));
+            tiled[i] = true;
+            left--;
+        }
+        if (left == 0) return MIMG_OK;
+    }
     for (int64_t r0 = 0; r0 < rows; r0 += 8) {
         const int64_t mr = rows - r0 < 8 ? rows - r0 : 8;
         ActPtrs c;
@@ -410,7 +427,7 @@ int matmul_quantized(const Weight* const* w, int count, const float* x, int64_t 
         c.ys16 = a.ys16 + r0 * R16;
         c.dbs = a.dbs + r0 * R32;
         c.ok = a.ok + r0;
-        bool done[3] = {false, false, false};
+        bool done[3] = {tiled[0], tiled[1], tiled[2]};
         for (int i = 0; i < count; i++) {
             if (done[i]) continue;
             hipError_t e;
@@ -433,12 +450,7 @@ int matmul_quantized(const Weight* const* w, int count, const float* x, int64_t 
                     e = launch_gemv_a8k(dws, n, c, mr, rows, x + r0 * K, bs, ys, s);
             } else {
                 const int64_t N = w[i]->dw.n;
-                if (w[i]->dw.dt == DT_Q8_0)
-                    e = launch_gemv_q8_0_a8(w[i]->dw, c, mr, rows, x + r0 * K, bias ? bias[i] : nullptr,
-                                            y[i] + r0 * N, N, s);
-                else
-                    e = launch_gemv_kq_a8_b32(w[i]->dw, c, mr, rows, x + r0 * K, bias ? bias[i] : nullptr,
-                                              y[i] + r0 * N, N, s);
+                e = launch_gemv_b32(w[i]->dw, c, mr, rows, x + r0 * K, bias ? bias[i] : nullptr, y[i] + r0 * N, s);
                 done[i] = true;
             }
             if (e != hipSuccess) return fail(MIMG_ERR_HIP, "product launch: %s", hipGetErrorString(e));
