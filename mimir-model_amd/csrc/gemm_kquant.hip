@@ -1,33 +1,27 @@
-// Prefill GEMM, Q4_K / Q6_K weights x 8-bit activations in blocks of 256
+// Prefill GEMM, Q6_K weights x 8-bit activations in blocks of 256
 // (dequant_matmul_a8.v2, block = 256) for many activation rows, on the int8
 // matrix cores (v_mfma_i32_32x32x32_i8). The result equals the decode GEMV's
 // bit for bit, as the reference's AMX/VNNI tile kernels equal its one-row
 // kernel (reference internal/kernels/amx.go:194-316, amx_test.go:41-141):
 // per (weight row n, activation row m) and block b the exact int32
-//   Q4_K  S = sum_k sc_s(k) q_k y_k,   M = sum_k m_s(k) y_k (= sum_s m_s xs_s)
-//   Q6_K  S = sum_k sc_s(k) (q_k - 32) y_k
-// then serially in block order tot = fma(f32(S), d*dx_b, tot) (and off for
-// Q4_K), result tot - off (+ bias), as dotQ8KRef (q8k_test.go:38-102).
+//   S = sum_k sc_s(k) (q_k - 32) y_k
+// then serially in block order tot = fma(f32(S), d*dx_b, tot), result tot
+// (+ bias), as dotQ8KRef (q8k_test.go:38-102). Q4_K has its own kernel
+// (gemm_q4k.hip); its layout, tried for Q6_K, measured 452 us against this
+// one's 424 at 4096 x 14336 x 2048 rows and 142 against 140 at 512 rows
+// (more to unpack a wave, and no two waves share the unpacked planes).
 //
-// Exact integer products on int8 MFMA: the scaled weight w = sc*q does not
-// fit int8 (Q4_K up to 945, Q6_K -4096..4064), so it is split in two planes.
-// Q4_K: sc = 8*sh + sl (sh, sl <= 7), planes sh*q and sl*q (each <= 105),
-// S = 8*sum(sh*q*y) + sum(sl*q*y); the planes are the packed nibbles times
-// a constant. Q6_K: w = 256*hi + lo with lo the low byte of w as a signed
-// value (-128..127) and hi in [-16, 16], S = 256*sum(hi*y) + sum(lo*y):
-// with u = w + 128 in a 16-bit lane, hi is u's high byte and lo its low
-// byte with the top bit flipped. Each MFMA sum is exact in int32 (|sum| <
-// 2^31 for 256-element blocks). Q4_K's M term = sum_s m_s xs_s comes from
-// the activation's per-32 sums xs: one v_mfma_f32_32x32x16_f16 a row tile
-// and block, with xs split as 64 hi + lo so that every operand is an exact
-// f16 and every partial sum an integer below 2^24 (measured on MI355X
-// against a third int8 plane with operand m_s over the 256 k: gate
-// M = 2048 525 -> 460 us, M = 512 122 -> 114 us).
+// Exact integer products on int8 MFMA: the scaled weight w = sc*q (-4096 ..
+// 4064) does not fit int8, so it is split in two planes, w = 256*hi + lo with
+// lo the low byte of w as a signed value (-128..127) and hi in [-16, 16],
+// S = 256*sum(hi*y) + sum(lo*y): with u = w + 128 in a 16-bit lane, hi is
+// u's high byte and lo its low byte with the top bit flipped. Each MFMA sum
+// is exact in int32 (|sum| < 2^31 for 256-element blocks).
 //
 // Operands: the activation rows are the MFMA's row operand and the weight
 // rows its column operand, so a lane of the 32 x 32 result holds one weight
 // row (lane l: row l % 32) and 16 activation rows (8j + 4(l/32) + r), and
-// needs one block scale d (and dmin) per block. A k step of 32 is one
+// needs one block scale d per block. A k step of 32 is one
 // sub-block; lane l supplies k 16(l/32)..+15 of it for both operands.
 //
 // Tiling: a workgroup of NW x WM waves owns 32 NW weight rows x 64 WM
@@ -50,34 +44,26 @@ namespace mimg {
 
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
-typedef float v16f __attribute__((ext_vector_type(16)));
-typedef _Float16 v8h __attribute__((ext_vector_type(8)));
-typedef _Float16 h2 __attribute__((ext_vector_type(2)));
 
 // Workgroup shape: NW waves along the weight rows (32 each), WM along the
 // activation rows (64 each: two MFMA row tiles).
-template <uint32_t DT, int NW, int WM>
+template <int NW, int WM>
 struct GemmLayout {
     static constexpr int T = 64 * NW * WM;   // threads
     static constexpr int BN = 32 * NW;       // weight rows per workgroup
     static constexpr int BM = 64 * WM;       // activation rows per workgroup
-    // LDS per weight row: a Q4_K block (16-byte aligned) as its 9 chunks of
-    // 16 bytes; a Q6_K block (2-byte aligned) as the 14 aligned chunks that
+    // LDS per weight row: a block (2-byte aligned) as the 14 aligned chunks that
     // cover it and one more, the block starting (address & 15) bytes into its
     // slot. The fifteenth chunk puts rows 60 dwords apart instead of 56: the
     // dword reads of 32 rows then meet each bank twice, not four times
     // (measured on MI355X: down M = 2048 509 -> 478 us).
-    static constexpr int WCH = DT == DT_Q4_K ? 9 : 15;
+    static constexpr int WCH = 15;
     static constexpr int WSLOT = 16 * WCH;
     static constexpr int WDMA = (BN * WCH + T - 1) / T;  // copies per thread per block
     static constexpr int WBYTES = WDMA * T * 16;         // incl. slack for unconditional copies
     static constexpr int ADMA = BM * 16 / T;
     static constexpr int ABYTES = BM * 256;
-    // Q4_K: the block's per-32 activation sums xs (eight int16, 16 bytes) of
-    // the BM rows, one copy per thread of a group of 256 (slots past BM:
-    // the last row again)
-    static constexpr int XBYTES = DT == DT_Q4_K ? 256 * 16 : 0;
-    static constexpr int BUF = WBYTES + ABYTES + XBYTES;
+    static constexpr int BUF = WBYTES + ABYTES;
     static constexpr int DXBYTES = T * 4;                // one dword copy per thread (BM used)
     static_assert(ADMA * T == BM * 16 && T >= BM && BM <= 256 && WM == 2, "GEMM tile shape");
 };
@@ -92,7 +78,6 @@ struct GemmArgs {
     int64_t K;
     const int8_t* q;       // [M][K]
     const float* d32;      // [M][K/32]
-    const int16_t* xs;     // [M][K/32]
     const int32_t* ok;     // [M]
     const float* x;        // [M][K] f32 (fallback)
     int fused;             // float32 fallback order (rows of the whole call <= 8)
@@ -140,9 +125,9 @@ __device__ __forceinline__ uint32_t q6k_slot_off(const GemmArgs& A, int n, int b
 
 // Issues the copies of block b into LDS buffer `buf` (every thread issues
 // exactly NDMA instructions, so the wait counts are the same in each wave).
-template <uint32_t DT, int NW, int WM>
+template <int NW, int WM>
 __device__ __forceinline__ void gemm_issue_block(const GemmArgs& A, int n0, int m0, int b, uint8_t* buf, uint8_t* dl) {
-    using L = GemmLayout<DT, NW, WM>;
+    using L = GemmLayout<NW, WM>;
     const int t = threadIdx.x, wave = t >> 6;
     uint8_t* wl = buf;
     uint8_t* al = buf + L::WBYTES;
@@ -151,8 +136,8 @@ __device__ __forceinline__ void gemm_issue_block(const GemmArgs& A, int n0, int 
         const int c = min(L::T * i + t, L::BN * L::WCH - 1);  // chunk of 16 bytes
         const int r = c / L::WCH, j = c - L::WCH * r;
         const int n = min(n0 + r, A.N - 1);
-        const uint8_t* blk = A.W + (int64_t)n * A.rb + (int64_t)b * (DT == DT_Q4_K ? Q4K_BYTES : Q6K_BYTES);
-        const uint8_t* base = DT == DT_Q4_K ? blk : (const uint8_t*)__builtin_align_down(blk, 16);
+        const uint8_t* blk = A.W + (int64_t)n * A.rb + (int64_t)b * Q6K_BYTES;
+        const uint8_t* base = (const uint8_t*)__builtin_align_down(blk, 16);
         lds_copy16(base + 16 * j, wl + 16 * (L::T * i + 64 * wave));
     }
 #pragma unroll
@@ -166,22 +151,16 @@ __device__ __forceinline__ void gemm_issue_block(const GemmArgs& A, int n0, int 
         const int m = min(m0 + min(t, L::BM - 1), A.M - 1);
         lds_copy4(A.d32 + (int64_t)m * (A.K / 32) + 8 * b, dl + 4 * (64 * wave));  // slots t >= BM are slack
     }
-    if constexpr (DT == DT_Q4_K) {
-        if (wave < 4) {
-            const int m = min(m0 + min(t, L::BM - 1), A.M - 1);
-            lds_copy16(A.xs + (int64_t)m * (A.K / 32) + 8 * b, al + L::ABYTES + 16 * (64 * wave));
-        }
-    }
 }
 
 // The same copies issued by the four trailing waves only (rank tr of 256),
 // during their half of the block that runs the float chain: the leading
 // waves' half holds the MFMAs and must not wait behind copy issue (measured
 // on MI355X at gate M = 2048: 4-7 % faster than every wave issuing its share).
-template <uint32_t DT, int NW, int WM>
+template <int NW, int WM>
 __device__ __forceinline__ void gemm_issue_block_tr(const GemmArgs& A, int n0, int m0, int b, uint8_t* buf, uint8_t* dl,
                                                     int tr) {
-    using L = GemmLayout<DT, NW, WM>;
+    using L = GemmLayout<NW, WM>;
     constexpr int T2 = 256, WD2 = (L::BN * L::WCH + T2 - 1) / T2, AD2 = L::BM * 16 / T2;
     static_assert(WD2 * T2 * 16 <= L::WBYTES && L::BM <= T2, "trailer copy layout");
     const int wt = tr >> 6;
@@ -192,8 +171,8 @@ __device__ __forceinline__ void gemm_issue_block_tr(const GemmArgs& A, int n0, i
         const int c = min(T2 * i + tr, L::BN * L::WCH - 1);
         const int r = c / L::WCH, j = c - L::WCH * r;
         const int n = min(n0 + r, A.N - 1);
-        const uint8_t* blk = A.W + (int64_t)n * A.rb + (int64_t)b * (DT == DT_Q4_K ? Q4K_BYTES : Q6K_BYTES);
-        const uint8_t* base = DT == DT_Q4_K ? blk : (const uint8_t*)__builtin_align_down(blk, 16);
+        const uint8_t* blk = A.W + (int64_t)n * A.rb + (int64_t)b * Q6K_BYTES;
+        const uint8_t* base = (const uint8_t*)__builtin_align_down(blk, 16);
         lds_copy16(base + 16 * j, wl + 16 * (T2 * i + 64 * wt));
     }
 #pragma unroll
@@ -207,10 +186,6 @@ __device__ __forceinline__ void gemm_issue_block_tr(const GemmArgs& A, int n0, i
         const int m = min(m0 + min(tr, L::BM - 1), A.M - 1);
         lds_copy4(A.d32 + (int64_t)m * (A.K / 32) + 8 * b, dl + 4 * (64 * wt));
     }
-    if constexpr (DT == DT_Q4_K) {
-        const int m = min(m0 + min(tr, L::BM - 1), A.M - 1);
-        lds_copy16(A.xs + (int64_t)m * (A.K / 32) + 8 * b, al + L::ABYTES + 16 * (64 * wt));
-    }
 }
 
 // 16 bytes at an LDS address that is 2-byte aligned: five aligned dwords
@@ -223,9 +198,9 @@ __device__ __forceinline__ u32x4 lds_read16_a2(const uint8_t* p) {
                  __builtin_amdgcn_alignbyte(w3, w2, sh), __builtin_amdgcn_alignbyte(w4, w3, sh)};
 }
 
-template <uint32_t DT, int NW, int WM>
-__global__ __launch_bounds__(64 * NW * WM) void gemm_a8k_kernel(GemmArgs A) {
-    using L = GemmLayout<DT, NW, WM>;
+template <int NW, int WM>
+__global__ __launch_bounds__(64 * NW * WM) void gemm_q6k_kernel(GemmArgs A) {
+    using L = GemmLayout<NW, WM>;
     __shared__ __align__(16) uint8_t smem[2 * L::BUF];
     __shared__ __align__(16) uint8_t dxs[3 * L::DXBYTES];
     __shared__ int flags[1];
@@ -262,12 +237,11 @@ __global__ __launch_bounds__(64 * NW * WM) void gemm_a8k_kernel(GemmArgs A) {
         if (f) flags[0] = 1;
     }
 
-    float tot[2][16], off[2][16];
+    float tot[2][16];
 #pragma unroll
-    for (int i = 0; i < 16; i++) tot[0][i] = tot[1][i] = off[0][i] = off[1][i] = 0.f;
+    for (int i = 0; i < 16; i++) tot[0][i] = tot[1][i] = 0.f;
     v16i accH[2], accL[2];
-    v16f accM[2];  // Q4_K: the mins term, exact integers in f32
-    float dN = 0.f, dminN = 0.f;
+    float dN = 0.f;
 
     // Block b's integer sums (the MFMAs) from LDS buffer b & 1.
     auto block_sums = [&](int b) {
@@ -279,124 +253,46 @@ __global__ __launch_bounds__(64 * NW * WM) void gemm_a8k_kernel(GemmArgs A) {
             const int row = 64 * wm + 32 * tt + a;
             return *(const v4i*)(al + row * 256 + 16 * ((2 * ks + g) ^ (row & 15)));
         };
-        if constexpr (DT == DT_Q4_K) {
-            const uint8_t* wr = wl + (32 * wn + a) * L::WSLOT;
-            const uint32_t dd = *(const uint32_t*)wr;
-            dN = f16_to_f32(dd & 0xFFFFu);
-            dminN = f16_to_f32(dd >> 16);
-            const uint32_t* sw = (const uint32_t*)(wr + 4);
-            const Q4KScales s = q4k_scales(sw[0], sw[1], sw[2]);
-            u32x4 qv[4];
+        const uint8_t* wr = wl + (32 * wn + a) * L::WSLOT + q6k_slot_off(A, nrow, b);
+        u32x4 qlv[4], qhv[2];
 #pragma unroll
-            for (int c = 0; c < 4; c++) qv[c] = *(const u32x4*)(wr + 16 + 32 * c + 16 * g);
+        for (int i = 0; i < 4; i++) qlv[i] = lds_read16_a2(wr + 64 * (i >> 1) + 32 * (i & 1) + 16 * g);
 #pragma unroll
-            for (int ks = 0; ks < 8; ks++) {
-                const v4i a0 = arow(ks, 0), a1 = arow(ks, 1);
-                const uint32_t sc = byte_of(s.sc, ks);
-                // sc = 8*sh + sl with sh, sl <= 7: sh*q and sl*q (q <= 15) are at
-                // most 105, so each plane is the packed nibbles times a small
-                // constant (16-bit lanes, no carry between the bytes).
-                const short sh = (short)(sc >> 3), sl = (short)(sc & 7);
-                const s16x2 shp = {sh, sh}, slp = {sl, sl};
-                const int shift = 4 * (ks & 1);  // sub-block 2c: low nibbles, 2c+1: high
-                const u32x4 qd = qv[ks >> 1];
-                v4i bH, bL;
+        for (int h = 0; h < 2; h++) qhv[h] = lds_read16_a2(wr + 128 + 32 * h + 16 * g);
+        const u32x4 scv = lds_read16_a2(wr + 192);
+        {
+            const uint32_t* dw = (const uint32_t*)__builtin_align_down(wr + 208, 4);
+            const uint32_t sh = (uint32_t)((uintptr_t)(wr + 208) & 3);
+            dN = f16_to_f32(__builtin_amdgcn_alignbyte(dw[1], dw[0], sh) & 0xFFFFu);
+        }
 #pragma unroll
-                for (int k = 0; k < 4; k++) {
-                    const s16x2 nib = as_s16x2((qd[k] >> shift) & 0x0F0F0F0Fu);
-                    bH[k] = (int)as_u32(nib * shp);
-                    bL[k] = (int)as_u32(nib * slp);
-                }
-                const v16i z = {};
-                accH[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a0, bH, ks ? accH[0] : z, 0, 0, 0);
-                accH[1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a1, bH, ks ? accH[1] : z, 0, 0, 0);
-                accL[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a0, bL, ks ? accL[0] : z, 0, 0, 0);
-                accL[1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a1, bL, ks ? accL[1] : z, 0, 0, 0);
+        for (int ks = 0; ks < 8; ks++) {
+            const v4i a0 = arow(ks, 0), a1 = arow(ks, 1);
+            const int h = ks >> 2, p = ks & 3;
+            const u32x4 ql = qlv[2 * h + (p & 1)], qh = qhv[h];
+            const int si = 8 * h + g + 2 * p;  // scale of this lane's 16 elements
+            const int sc = (int)(int8_t)(uint8_t)(scv[si >> 2] >> (8 * (si & 3)));
+            // u = sc*q - 32*sc + 128 = w + 128 in 16-bit lanes (packed
+            // integer multiply-add, exact: |u| <= 4224)
+            const short cu = (short)(128 - 32 * sc);
+            const s16x2 sc2 = {(short)sc, (short)sc}, c2 = {cu, cu};
+            v4i bH, bL;
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                const uint32_t q6 = (((p >> 1) ? (ql[k] >> 4) : ql[k]) & 0x0F0F0F0Fu) |
+                                    (((qh[k] >> (2 * p)) & 0x03030303u) << 4);
+                const uint32_t ue = as_u32(as_s16x2(__builtin_amdgcn_perm(0u, q6, 0x0C020C00u)) * sc2 + c2);
+                const uint32_t uo = as_u32(as_s16x2(__builtin_amdgcn_perm(0u, q6, 0x0C030C01u)) * sc2 + c2);
+                // v_perm selector [src1.bX, src0.bX, src1.bY, src0.bY]: the
+                // high bytes of the lanes (hi) and the low bytes (lo + 128)
+                bH[k] = (int)__builtin_amdgcn_perm(uo, ue, 0x07030501u);
+                bL[k] = (int)(__builtin_amdgcn_perm(uo, ue, 0x06020400u) ^ 0x80808080u);
             }
-            // The mins term M = sum_s m_s xs_s of every (weight row,
-            // activation row) on one f16 MFMA a row tile (k = 16: the eight
-            // sub-blocks twice). xs = 64 hi + lo with hi in [-64, 63] and lo
-            // in [0, 63]: the row operand holds hi_s at k = s (lanes g = 0)
-            // and lo_s at k = 8 + s (g = 1), the weight operand 64 m_s and
-            // m_s. Every product and partial sum is an integer below 2^24,
-            // so the f32 result is M exactly. The f16 values are built as
-            // f16(1024 + v) from the bits 0x6400 + v, minus 1024.
-            {
-                const uint32_t mw[2] = {(uint32_t)s.m, (uint32_t)(s.m >> 32)};
-                const h2 mul = g ? h2{(_Float16)1.0f, (_Float16)1.0f} : h2{(_Float16)64.0f, (_Float16)64.0f};
-                const h2 c1024 = {(_Float16)1024.0f, (_Float16)1024.0f};
-                v8h bm;
-#pragma unroll
-                for (int j = 0; j < 4; j++) {
-                    const uint32_t u = __builtin_amdgcn_perm(0u, mw[j >> 1], (j & 1) ? 0x0C030C02u : 0x0C010C00u);
-                    const h2 f = (__builtin_bit_cast(h2, u | 0x64006400u) - c1024) * mul;
-                    bm[2 * j] = f.x;
-                    bm[2 * j + 1] = f.y;
-                }
-                const uint8_t* xl = al + L::ABYTES;
-                const short sh = g ? 0 : 6;
-                const s16x2 sh2 = {sh, sh};
-                const uint32_t msk = g ? 0x003F003Fu : 0xFFFFFFFFu;
-                const h2 cf = g ? c1024 : h2{(_Float16)1088.0f, (_Float16)1088.0f};
-                const s16x2 cadd = g ? s16x2{0x6400, 0x6400} : s16x2{0x6440, 0x6440};
-#pragma unroll
-                for (int tt = 0; tt < 2; tt++) {
-                    const u32x4 xw = *(const u32x4*)(xl + 16 * (64 * wm + 32 * tt + a));
-                    const uint32_t xd[4] = {xw.x, xw.y, xw.z, xw.w};
-                    v8h av;
-#pragma unroll
-                    for (int j = 0; j < 4; j++) {
-                        const uint32_t v = as_u32(as_s16x2(xd[j]) >> sh2) & msk;
-                        const h2 f = __builtin_bit_cast(h2, as_u32(as_s16x2(v) + cadd)) - cf;
-                        av[2 * j] = f.x;
-                        av[2 * j + 1] = f.y;
-                    }
-                    const v16f zf = {};
-                    accM[tt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(av, bm, zf, 0, 0, 0);
-                }
-            }
-        } else {
-            const uint8_t* wr = wl + (32 * wn + a) * L::WSLOT + q6k_slot_off(A, nrow, b);
-            u32x4 qlv[4], qhv[2];
-#pragma unroll
-            for (int i = 0; i < 4; i++) qlv[i] = lds_read16_a2(wr + 64 * (i >> 1) + 32 * (i & 1) + 16 * g);
-#pragma unroll
-            for (int h = 0; h < 2; h++) qhv[h] = lds_read16_a2(wr + 128 + 32 * h + 16 * g);
-            const u32x4 scv = lds_read16_a2(wr + 192);
-            {
-                const uint32_t* dw = (const uint32_t*)__builtin_align_down(wr + 208, 4);
-                const uint32_t sh = (uint32_t)((uintptr_t)(wr + 208) & 3);
-                dN = f16_to_f32(__builtin_amdgcn_alignbyte(dw[1], dw[0], sh) & 0xFFFFu);
-            }
-#pragma unroll
-            for (int ks = 0; ks < 8; ks++) {
-                const v4i a0 = arow(ks, 0), a1 = arow(ks, 1);
-                const int h = ks >> 2, p = ks & 3;
-                const u32x4 ql = qlv[2 * h + (p & 1)], qh = qhv[h];
-                const int si = 8 * h + g + 2 * p;  // scale of this lane's 16 elements
-                const int sc = (int)(int8_t)(uint8_t)(scv[si >> 2] >> (8 * (si & 3)));
-                // u = sc*q - 32*sc + 128 = w + 128 in 16-bit lanes (packed
-                // integer multiply-add, exact: |u| <= 4224)
-                const short cu = (short)(128 - 32 * sc);
-                const s16x2 sc2 = {(short)sc, (short)sc}, c2 = {cu, cu};
-                v4i bH, bL;
-#pragma unroll
-                for (int k = 0; k < 4; k++) {
-                    const uint32_t q6 = (((p >> 1) ? (ql[k] >> 4) : ql[k]) & 0x0F0F0F0Fu) |
-                                        (((qh[k] >> (2 * p)) & 0x03030303u) << 4);
-                    const uint32_t ue = as_u32(as_s16x2(__builtin_amdgcn_perm(0u, q6, 0x0C020C00u)) * sc2 + c2);
-                    const uint32_t uo = as_u32(as_s16x2(__builtin_amdgcn_perm(0u, q6, 0x0C030C01u)) * sc2 + c2);
-                    // v_perm selector [src1.bX, src0.bX, src1.bY, src0.bY]: the
-                    // high bytes of the lanes (hi) and the low bytes (lo + 128)
-                    bH[k] = (int)__builtin_amdgcn_perm(uo, ue, 0x07030501u);
-                    bL[k] = (int)(__builtin_amdgcn_perm(uo, ue, 0x06020400u) ^ 0x80808080u);
-                }
-                const v16i z = {};
-                accH[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a0, bH, ks ? accH[0] : z, 0, 0, 0);
-                accH[1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a1, bH, ks ? accH[1] : z, 0, 0, 0);
-                accL[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a0, bL, ks ? accL[0] : z, 0, 0, 0);
-                accL[1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a1, bL, ks ? accL[1] : z, 0, 0, 0);
-            }
+            const v16i z = {};
+            accH[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a0, bH, ks ? accH[0] : z, 0, 0, 0);
+            accH[1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a1, bH, ks ? accH[1] : z, 0, 0, 0);
+            accL[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a0, bL, ks ? accL[0] : z, 0, 0, 0);
+            accL[1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a1, bL, ks ? accL[1] : z, 0, 0, 0);
         }
     };
     // Block b's float step, per output in block order: lane l holds
@@ -412,9 +308,8 @@ __global__ __launch_bounds__(64 * NW * WM) void gemm_a8k_kernel(GemmArgs A) {
 #pragma unroll
                 for (int r = 0; r < 4; r++) {
                     const int i = 4 * j + r;
-                    const int S = (accH[tt][i] << (DT == DT_Q4_K ? 3 : 8)) + accL[tt][i];
+                    const int S = (accH[tt][i] << 8) + accL[tt][i];
                     tot[tt][i] = __builtin_fmaf((float)S, dN * dxr[r], tot[tt][i]);
-                    if constexpr (DT == DT_Q4_K) off[tt][i] = __builtin_fmaf(accM[tt][i], dminN * dxr[r], off[tt][i]);
                 }
             }
         }
@@ -427,13 +322,13 @@ __global__ __launch_bounds__(64 * NW * WM) void gemm_a8k_kernel(GemmArgs A) {
     // Buffer (b+1) & 1 was last read by the trailing waves' sums of block
     // b-1, before the barrier that starts block b's first half; dx stage
     // (b+1) % 3 by the chain of block b-2.
-    gemm_issue_block<DT, NW, WM>(A, n0, m0, 0, smem, dxs);
+    gemm_issue_block<NW, WM>(A, n0, m0, 0, smem, dxs);
     GM_WAIT_VMCNT(0);
     gm_barrier();
     for (int b = 0; b <= nb; b++) {
         // first half: the leaders' sums of block b, the trailers' chain of b-1
         if (b + 1 < nb && !leader)
-            gemm_issue_block_tr<DT, NW, WM>(A, n0, m0, b + 1, smem + ((b + 1) & 1) * L::BUF,
+            gemm_issue_block_tr<NW, WM>(A, n0, m0, b + 1, smem + ((b + 1) & 1) * L::BUF,
                                             dxs + ((b + 1) % 3) * L::DXBYTES, trank);
         if (leader) {
             if (b < nb) block_sums(b);
@@ -463,7 +358,7 @@ __global__ __launch_bounds__(64 * NW * WM) void gemm_a8k_kernel(GemmArgs A) {
                 const int m = m0 + 64 * wm + 32 * tt + 8 * (i >> 2) + 4 * g + (i & 3);
                 if (m >= A.M) continue;
                 if (refused && A.ok[m] == 0) continue;
-                float res = DT == DT_Q4_K ? tot[tt][i] - off[tt][i] : tot[tt][i];
+                float res = tot[tt][i];
                 if (A.bias) res += bn;
                 A.y[(int64_t)m * A.N + n] = res;
             }
@@ -477,7 +372,7 @@ __global__ __launch_bounds__(64 * NW * WM) void gemm_a8k_kernel(GemmArgs A) {
         const int nn = n0 + pidx % L::BN, m = m0 + pidx / L::BN;
         if (nn >= A.N || m >= A.M) continue;
         if (A.wref[nn] == 0 && A.ok[m] != 0) continue;
-        float res = f32dot_g8<DT>(A.W + (int64_t)nn * A.rb, A.x + (int64_t)m * A.K, A.K, A.fused != 0);
+        float res = f32dot_g8<DT_Q6_K>(A.W + (int64_t)nn * A.rb, A.x + (int64_t)m * A.K, A.K, A.fused != 0);
         if (A.bias) res += A.bias[nn];
         if ((t & 7) == 0) A.y[(int64_t)m * A.N + nn] = res;
     }
@@ -490,6 +385,11 @@ bool gemm_a8k_ok(const DevWeight& w) {
 hipError_t launch_gemm_a8k(const DevWeight& w, const ActPtrs& a, int64_t rows, int64_t total_rows, const float* x,
                            const float* bias, float* y, hipStream_t stream) {
     if (!gemm_a8k_ok(w) || rows <= 0 || rows > (1 << 30) || w.n > (1 << 30)) return hipErrorInvalidValue;
+    if (w.dt == DT_Q4_K) {
+        hipError_t e = hipSuccess;
+        if (launch_gemm_q4k(w, a, rows, total_rows, x, bias, y, stream, &e)) return e;
+        return launch_gemm_a8k_16(w, a, rows, total_rows, x, bias, y, stream);
+    }
     GemmArgs A;
     A.W = w.data;
     A.wref = w.wref;
@@ -502,23 +402,21 @@ hipError_t launch_gemm_a8k(const DevWeight& w, const ActPtrs& a, int64_t rows, i
     A.K = w.k;
     A.q = a.q;
     A.d32 = a.d32;
-    A.xs = a.xs;
     A.ok = a.ok;
     A.x = x;
     A.fused = total_rows <= 8;
     // 128 weight rows x 128 activation rows per workgroup of eight waves;
     // where that leaves CUs without a workgroup (few weight or activation
     // rows: down at 512 rows, 64 prompt rows) the 16 x 16 x 64 kernel with
-    // 64-row tiles runs instead (measured on MI355X: gate/down at 64 rows
-    // 41/155 against 57/218 us, down at 512 rows 176 against 222 us).
+    // 64-row tiles runs instead (measured on MI355X: down at 512 rows 176
+    // against 222 us).
     constexpr int BN = 128, BM = 128;
     A.tiles_m = (int)((rows + BM - 1) / BM);
     const int64_t nwg = (w.n + BN - 1) / BN * A.tiles_m;
     if (nwg < 256) return launch_gemm_a8k_16(w, a, rows, total_rows, x, bias, y, stream);
     if (nwg > 0x7fffffff) return hipErrorInvalidValue;
     const dim3 grid((unsigned)nwg), block(512);
-    if (w.dt == DT_Q4_K) hipLaunchKernelGGL((gemm_a8k_kernel<DT_Q4_K, 4, 2>), grid, block, 0, stream, A);
-    else hipLaunchKernelGGL((gemm_a8k_kernel<DT_Q6_K, 4, 2>), grid, block, 0, stream, A);
+    hipLaunchKernelGGL((gemm_q6k_kernel<4, 2>), grid, block, 0, stream, A);
     return hipGetLastError();
 }
 

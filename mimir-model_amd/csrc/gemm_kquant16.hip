@@ -654,21 +654,23 @@ __global__ __launch_bounds__(256) void gemm_a8k_ks_kernel(GemmArgs A) {
 
 }  // namespace g16
 
-template <class C>
-static hipError_t launch_g16(const g16::GemmArgs& A, uint32_t dt, int64_t n, int64_t rows, hipStream_t stream) {
+template <uint32_t DT, class C>
+static hipError_t launch_g16(const g16::GemmArgs& A, int64_t n, int64_t rows, hipStream_t stream) {
     using namespace g16;
     const dim3 grid((unsigned)((n + C::BN - 1) / C::BN), (unsigned)((rows + C::BM - 1) / C::BM));
-    if (dt == DT_Q4_K)
-        hipLaunchKernelGGL((gemm_a8k_kernel<DT_Q4_K, C>), grid, dim3(C::T), 0, stream, A);
-    else
-        hipLaunchKernelGGL((gemm_a8k_kernel<DT_Q6_K, C>), grid, dim3(C::T), 0, stream, A);
+    hipLaunchKernelGGL((gemm_a8k_kernel<DT, C>), grid, dim3(C::T), 0, stream, A);
     return hipGetLastError();
+}
+static hipError_t launch_g16_m64n32(const g16::GemmArgs& A, uint32_t dt, int64_t n, int64_t rows, hipStream_t stream) {
+    if (dt == DT_Q4_K) return launch_g16<DT_Q4_K, g16::CfgM64N32>(A, n, rows, stream);
+    return launch_g16<DT_Q6_K, g16::CfgM64N32>(A, n, rows, stream);
 }
 
 // The 16 x 16 x 64 form of the prefill GEMM (see the top of this file).
 // Up to 64 activation rows: 64-row tiles, 32 weight rows a workgroup where
 // that gives at least 256 workgroups, else 16; more rows: 64 x 128 tiles,
-// or 32 x 64 tiles where those give fewer than 256 workgroups.
+// or 32 x 64 tiles where those give fewer than 256 workgroups (Q4_K: always;
+// its larger grids are gemm_q4k.hip's).
 hipError_t launch_gemm_a8k_16(const DevWeight& w, const ActPtrs& a, int64_t rows, int64_t total_rows, const float* x,
                            const float* bias, float* y, hipStream_t stream) {
     using namespace g16;
@@ -689,7 +691,7 @@ hipError_t launch_gemm_a8k_16(const DevWeight& w, const ActPtrs& a, int64_t rows
     A.x = x;
     A.fused = total_rows <= 8;
     if (rows <= 64) {
-        if ((w.n + 31) / 32 >= 256) return launch_g16<CfgM64N32>(A, w.dt, w.n, rows, stream);
+        if ((w.n + 31) / 32 >= 256) return launch_g16_m64n32(A, w.dt, w.n, rows, stream);
         // 32-row tiles up to 32 rows (down at 32 rows: 51.5 against 61.4 us
         // with 64-row tiles), 64-row tiles above (62.4 against 65.7 us at 64
         // rows: the 32-row tiles read each weight twice)
@@ -708,8 +710,9 @@ hipError_t launch_gemm_a8k_16(const DevWeight& w, const ActPtrs& a, int64_t rows
     // 8B prompt of 512 rows 24.5 -> 23.3 ms; the same tiles for q, o and
     // down at 512 rows, 256 workgroups of 64 x 128, made it 25.6 ms, and
     // 16 x 64 tiles 33.0 ms)
-    if ((w.n + 63) / 64 * ((rows + 127) / 128) < 256) return launch_g16<CfgM64N32>(A, w.dt, w.n, rows, stream);
-    return launch_g16<CfgWide>(A, w.dt, w.n, rows, stream);
+    if (w.dt == DT_Q4_K || (w.n + 63) / 64 * ((rows + 127) / 128) < 256)
+        return launch_g16_m64n32(A, w.dt, w.n, rows, stream);
+    return launch_g16<DT_Q6_K, CfgWide>(A, w.n, rows, stream);
 }
 
 }  // namespace mimg

@@ -121,8 +121,12 @@ struct QaSetArgs {
 hipError_t launch_quantize_act_set(const QaSetArgs& a, int wgs, hipStream_t stream);
 
 // Many activation rows (already quantized) against one Q4_K/Q6_K matrix,
-// on the int8 matrix cores (gemm_kquant.hip); bit-identical to the GEMV.
+// on the int8 matrix cores (gemm_kquant.hip, gemm_q4k.hip); bit-identical to
+// the GEMV.
 bool gemm_a8k_ok(const DevWeight& w);
+// Q4_K's tiles (gemm_q4k.hip); false where the grid would be too small for them.
+bool launch_gemm_q4k(const DevWeight& w, const ActPtrs& a, int64_t rows, int64_t total_rows, const float* x,
+                     const float* bias, float* y, hipStream_t stream, hipError_t* err);
 // The 16 x 16 x 64 form for small grids (gemm_kquant16.hip); launch_gemm_a8k
 // picks it by grid size.
 hipError_t launch_gemm_a8k_16(const DevWeight& w, const ActPtrs& a, int64_t rows, int64_t total_rows, const float* x,

@@ -1,0 +1,45 @@
+"""Q4_K prefill tiles (gemm_q4k.hip): 128 weight rows by 32 activation rows
+from 96 workgroups of those, by 64 above 256 workgroups; bit for bit the
+oracle, at the edges of both tiles, on both sides of the rules, with bias and
+refusals (reference amx_test.go:41-141)."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+Q4_K = 66
+
+
+def check(gpu, oracle, rows, n, k, edit=None, bias=False):
+    wb = oracle.synthetic_weight(Q4_K, n, k, seed=rows + n)
+    x = oracle.synthetic_acts(rows, k, seed=rows + 1)
+    if edit:
+        edit(wb, x)
+    b = oracle.synthetic_acts(1, n, seed=rows + 2)[0] if bias else None
+    W = gpu.Weight(wb, Q4_K, n, k)
+    got = gpu.dequant_matmul_a8(W, x, bias=b, block=256)
+    W.release()
+    want = oracle.linear_a8(x, wb, Q4_K, n, k, bias=b, block=256, threads=8)
+    same = (got.view(np.uint32) == want.view(np.uint32)) | (np.isnan(got) & np.isnan(want))
+    assert same.all(), f"{(~same).sum()} of {same.size} differ, first at {np.argwhere(~same)[0]}"
+
+
+# 95 and 96 tiles of 32 rows, 256 and 272 tiles of 64 rows, a lone last row of
+# a tile in each direction, one block and several
+@pytest.mark.parametrize("rows,n,k", [(31, 12160, 256), (31, 12161, 512), (32, 12289, 256), (97, 3073, 768),
+                                      (96, 4096, 1024), (1024, 2048, 256), (1025, 2048, 512), (65, 16513, 256),
+                                      (2047, 1025, 1024)])
+def test_tiles_and_rules(gpu, oracle, rows, n, k):
+    check(gpu, oracle, rows, n, k, bias=rows % 2 == 1)
+
+
+@pytest.mark.parametrize("rows,n", [(100, 3100), (300, 7000)])
+def test_refusals(gpu, oracle, rows, n):
+    def edit(wb, x):
+        blocks = wb.reshape(n, 2, 144)
+        blocks[5, 0, 2:4] = (0x00, 0x7C)          # dmin = inf
+        blocks[n - 1, 1, 0:2] = (0x01, 0x7E)      # d = NaN
+        x[7, 3] = np.nan
+        x[rows - 1, 100] = np.float32(1e30)
+
+    check(gpu, oracle, rows, n, 512, edit=edit, bias=True)
