@@ -16,6 +16,22 @@ __host__ __device__ __forceinline__ int64_t vcache_at(int hk, int64_t j, int d, 
     return (((int64_t)hk * ((C + 7) >> 3) + (j >> 3)) * D + d) * 8 + (j & 7);
 }
 
+// The cache entries query t sees: k0 .. k0 + n - 1 of its kv head, from
+// kstart[t] (0 when null) to kend[t], clipped to the cache row and to maxk.
+struct AttRange {
+    int64_t k0, n;
+};
+__device__ __forceinline__ AttRange att_range(const int64_t* kend, const int64_t* kstart, int t, int64_t C,
+                                              int64_t maxk) {
+    AttRange r;
+    r.k0 = kstart ? (kstart[t] < 0 ? 0 : (kstart[t] >= C ? C - 1 : kstart[t])) : 0;
+    int64_t n = kend[t] + 1 - r.k0;
+    if (n > C - r.k0) n = C - r.k0;
+    if (n > maxk) n = maxk;
+    r.n = n < 0 ? 0 : n;
+    return r;
+}
+
 // The value of lane i ^ M (M a power of two below 64): DPP within a row of
 // 16 lanes for M <= 8 (quad permutes for 1 and 2; row shifts of four into
 // each half-row, by bank mask, for 4; a rotation by eight for 8), a

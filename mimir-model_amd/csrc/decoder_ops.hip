@@ -259,20 +259,6 @@ __global__ void rope_kv_kernel(float* __restrict__ q, const float* __restrict__ 
 // reference's scalar loop ends in NaN then); no visible key gives zeros.
 constexpr int ATT_MAXC = 8192;
 
-struct AttRange {
-    int64_t k0, n;
-};
-__device__ __forceinline__ AttRange att_range(const int64_t* kend, const int64_t* kstart, int t, int64_t C,
-                                              int64_t maxk) {
-    AttRange r;
-    r.k0 = kstart ? (kstart[t] < 0 ? 0 : (kstart[t] >= C ? C - 1 : kstart[t])) : 0;
-    int64_t n = kend[t] + 1 - r.k0;
-    if (n > C - r.k0) n = C - r.k0;
-    if (n > maxk) n = maxk;
-    r.n = n < 0 ? 0 : n;
-    return r;
-}
-
 template <bool F16>
 __device__ __forceinline__ float kv_load(const void* c, int64_t i) {
     if constexpr (F16) return (float)((const _Float16*)c)[i];
@@ -1272,347 +1258,6 @@ hipError_t launch_kv_store(const float* k, const float* v, const int64_t* pos, i
     return hipGetLastError();
 }
 
-// Prompt scores with a key per lane (many queries over one sequence): a
-// workgroup per (tiles of 256 cache entries, head, QG queries): the tiles
-// from the first entry any of its queries sees, blockIdx.x, gridDim.x
-// apart; thread i holds the key of cache entry kb + i (D values, f16 or
-// f32, in registers) and the QG query rows sit in LDS, read as broadcasts. For each query the lane runs
-// the reference's eight chains itself, l_c = fma(q[8m + c], k[8m + c], l_c)
-// for m = 0..D/8-1 in order, and combines them with the pairing
-// att_reduce8 uses (((l0+l1)+(l2+l3))+((l4+l5)+(l6+l7)) for keys in the
-// groups of four, ((l0+l4)+(l1+l5))+((l2+l6)+(l3+l7)) for the last n % 4):
-// the same operations on the same values as att_scores_kernel, so the same
-// bits, without its eight-lane split (sixteen 2-byte loads and a DPP
-// reduction per key and query). A wave skips a query none of its 64 keys is
-// visible to; stores are consecutive keys.
-// A value every lane holds the same copy of (read from LDS), made a scalar
-// so that comparisons on it are scalar branches, not exec masks.
-__device__ __forceinline__ int64_t uni64(int64_t x) {
-    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)x), hi = __builtin_amdgcn_readfirstlane((uint32_t)(x >> 32));
-    return (int64_t)(((uint64_t)hi << 32) | lo);
-}
-
-constexpr int ATT_KPL_QG = 32;
-
-template <bool F16, int D>
-__global__ __launch_bounds__(256) void att_scores_kpl_kernel(const float* __restrict__ q, const void* kc,
-                                                             const int64_t* __restrict__ kend,
-                                                             const int64_t* __restrict__ kstart, int T, int H,
-                                                             int Hkv, int64_t C, int64_t maxk,
-                                                             float* __restrict__ ws) {
-    constexpr int QG = ATT_KPL_QG, DM = D / 8;
-    constexpr int KW = F16 ? D / 2 : D;  // 32-bit words of a key
-    __shared__ __align__(16) float qs[QG * D];
-    __shared__ int64_t k0s[QG], ns[QG];
-    const int h = blockIdx.y, tid = threadIdx.x, w = tid >> 6;
-    const int hk = h / (H / Hkv), t0 = (int)blockIdx.z * QG;
-    if (tid < QG) {
-        const int t = t0 + tid;
-        const AttRange r = t < T ? att_range(kend, kstart, t, C, maxk) : AttRange{0, 0};
-        k0s[tid] = r.k0;
-        ns[tid] = r.n;
-    }
-    __syncthreads();
-    // the cache entries the queries see: [kmin, kfin); this workgroup takes
-    // the tiles of 256 of them from tile blockIdx.x, gridDim.x apart
-    int64_t kmin = INT64_MAX, kfin = 0;
-#pragma unroll
-    for (int i = 0; i < QG; i++) {
-        const int64_t ni = uni64(ns[i]), ki = uni64(k0s[i]);
-        if (ni <= 0) continue;
-        kmin = ki < kmin ? ki : kmin;
-        kfin = ki + ni > kfin ? ki + ni : kfin;
-    }
-    if (kfin == 0) return;  // uniform: no query sees a key
-    // the query rows (zeros past T: never stored)
-    for (int i = tid; i < QG * D / 4; i += 256) {
-        const int tq = i / (D / 4), d4 = i - tq * (D / 4), t = t0 + tq;
-        const float4 v = t < T ? *(const float4*)(q + ((int64_t)t * H + h) * D + 4 * d4) : float4{0.f, 0.f, 0.f, 0.f};
-        *(float4*)(qs + tq * D + 4 * d4) = v;
-    }
-    __syncthreads();
-    for (int64_t kb = kmin + 256 * (int64_t)blockIdx.x; kb < kfin; kb += 256 * (int64_t)gridDim.x) {
-    // this lane's key (entries past the cache read the last one, unstored)
-    const int64_t a = kb + tid, ac = a < C ? a : C - 1;
-    uint32_t kw[KW];
-    {
-        const uint4* kp = (const uint4*)((const uint8_t*)kc + ((int64_t)hk * C + ac) * D * (F16 ? 2 : 4));
-#pragma unroll
-        for (int i = 0; i < KW / 4; i++) {
-            const uint4 v = kp[i];
-            kw[4 * i] = v.x;
-            kw[4 * i + 1] = v.y;
-            kw[4 * i + 2] = v.z;
-            kw[4 * i + 3] = v.w;
-        }
-    }
-    const float scale = (float)(1.0 / sqrt((double)D));
-    const int64_t wa = kb + 64 * w;  // this wave's first cache entry
-    for (int i = 0; i < QG; i++) {
-        const int64_t k0 = uni64(k0s[i]), n = uni64(ns[i]);
-        if (n <= 0 || k0 >= wa + 64 || k0 + n <= wa) continue;  // uniform
-        const float* qr = qs + i * D;
-        float l[8];
-#pragma unroll
-        for (int c = 0; c < 8; c++) l[c] = 0.f;
-#pragma unroll
-        for (int m = 0; m < DM; m++) {
-            const float4 qa = *(const float4*)(qr + 8 * m), qb = *(const float4*)(qr + 8 * m + 4);
-            const float qv[8] = {qa.x, qa.y, qa.z, qa.w, qb.x, qb.y, qb.z, qb.w};
-#pragma unroll
-            for (int c = 0; c < 8; c++) {
-                float kv;
-                if constexpr (F16) {
-                    const uint32_t wd = kw[4 * m + c / 2];
-                    kv = (float)__builtin_bit_cast(_Float16, (uint16_t)((c & 1) ? wd >> 16 : wd & 0xFFFF));
-                } else {
-                    kv = __uint_as_float(kw[8 * m + c]);
-                }
-                l[c] = __builtin_fmaf(qv[c], kv, l[c]);
-            }
-        }
-        const int64_t j = a - k0, n4 = n - n % 4;
-        const float pf = ((l[0] + l[1]) + (l[2] + l[3])) + ((l[4] + l[5]) + (l[6] + l[7]));
-        const float pn = ((l[0] + l[4]) + (l[1] + l[5])) + ((l[2] + l[6]) + (l[3] + l[7]));
-        const float p = j < n4 ? pf : pn;
-        if (j >= 0 && j < n) ws[((int64_t)(t0 + i) * H + h) * maxk + j] = p * scale;
-    }
-    }
-}
-
-// Prompt weighted sum with queries' chains side by side: a workgroup per
-// (head, QG queries) of D/64 x QG/QW waves; a wave takes 64 dims of the head
-// and QW of the queries, each lane the QW chains acc_q = fma(e_q[j],
-// v_j[d], acc_q) of its dim in key order (the same chains as
-// att_wsum_q4_kernel, which gives a wave one query: here QW independent
-// fmas follow each value, so the chains' latency is hidden). The value of
-// key j is read straight from the blocked cache (one 16-byte load gives
-// eight keys of the dim), four blocks ahead; a block's weights are read
-// from LDS before its fmas. Per query first: max and NaN check over its
-// scores, e = Cephes exp(s - max) for the first n & ~7 keys and the f64 exp
-// for the rest, into LDS as [key][query]; the eight stride-8 lane sums in
-// key order, ((s0+s4)+(s1+s5))+((s2+s6)+(s3+s7)) and the rest in order;
-// o[d] = acc / sum (NaN for a NaN score or an infinite max, 0 for no
-// visible key). Queries that do not share the first visible entry run in
-// passes of one.
-constexpr int ATT_QPL_QG = 16, ATT_QPL_QW = 8;
-
-template <bool F16, int D>
-__global__ __launch_bounds__(D * ATT_QPL_QG / ATT_QPL_QW) void att_wsum_qpl_kernel(
-    const void* vc, const int64_t* __restrict__ kend, const int64_t* __restrict__ kstart, int T, int H, int Hkv,
-    int64_t C, int64_t maxk, const float* __restrict__ ws, float* __restrict__ out) {
-    constexpr int QG = ATT_QPL_QG, QW = ATT_QPL_QW, DH = D / 64, NT = D * QG / QW, NWV = NT / 64;
-    using VT = typename std::conditional<F16, _Float16, float>::type;
-    extern __shared__ __align__(16) float ew[];  // [maxk][QG]
-    __shared__ int64_t k0s[QG], ns[QG];
-    __shared__ float sums[QG];
-    __shared__ int bads[QG];
-    __shared__ float mxs[NWV][QG];
-    __shared__ int bws[NWV][QG];
-    const int h = blockIdx.y, t = threadIdx.x, w = t >> 6, lane = t & 63;
-    const int d = lane + 64 * (w % DH), qg = w / DH;  // this lane's dim and query group
-    const int hk = h / (H / Hkv), t0 = (int)blockIdx.z * QG;
-    if (t < QG) {
-        const int tq = t0 + t;
-        const AttRange r = tq < T ? att_range(kend, kstart, tq, C, maxk) : AttRange{0, 0};
-        k0s[t] = r.k0;
-        ns[t] = r.n;
-    }
-    __syncthreads();
-    // 1. Every query's scores into LDS ([key][query]), eight loads a thread
-    // in flight (the index space is QG rows of a power-of-two length, so a
-    // row and a key are a shift and a mask); then max, NaN check and the
-    // exps in place, thread t on query t % QG and keys t / QG + k NT / QG (so
-    // consecutive threads touch consecutive words), the maxima and the NaN
-    // flags combined across the threads of a query.
-    int64_t nall = 0;
-#pragma unroll
-    for (int i = 0; i < QG; i++) nall = ns[i] > nall ? ns[i] : nall;
-    int lg = 0;
-    while ((1ll << lg) < nall) lg++;
-    const int64_t span = (int64_t)QG << lg;
-    for (int64_t b0 = t; b0 < (nall > 0 ? span : 0); b0 += 8 * NT) {
-        float v[8];
-#pragma unroll
-        for (int u = 0; u < 8; u++) {
-            const int64_t idx = b0 + (int64_t)NT * u;
-            const int qi = (int)(idx >> lg) & (QG - 1);
-            const int64_t j = idx & ((1ll << lg) - 1);
-            const bool ok = idx < span && j < ns[qi];
-            v[u] = ok ? ws[((int64_t)(t0 + qi) * H + h) * maxk + j] : 0.f;
-        }
-#pragma unroll
-        for (int u = 0; u < 8; u++) {
-            const int64_t idx = b0 + (int64_t)NT * u;
-            const int qi = (int)(idx >> lg) & (QG - 1);
-            const int64_t j = idx & ((1ll << lg) - 1);
-            if (idx < span && j < ns[qi]) ew[j * QG + qi] = v[u];
-        }
-    }
-    __syncthreads();
-    {
-        constexpr int JS = NT / QG;  // keys a step
-        const int qi = t & (QG - 1), jj = t / QG;
-        const int64_t n = ns[qi];
-        float mx = -INFINITY;
-        int bad = 0;
-        for (int64_t j = jj; j < n; j += JS) {
-            const float v = ew[j * QG + qi];
-            bad |= v != v;
-            mx = fmaxf(mx, v);
-        }
-        // the threads of query qi: lanes qi + 16m of each wave, then the waves
-        mx = fmaxf(mx, lane_xor_f32<16>(mx));
-        mx = fmaxf(mx, lane_xor_f32<32>(mx));
-        bad |= __shfl_xor(bad, 16);
-        bad |= __shfl_xor(bad, 32);
-        if (lane < QG) {
-            mxs[w][lane] = mx;
-            bws[w][lane] = bad;
-        }
-        __syncthreads();
-#pragma unroll
-        for (int i = 0; i < NWV; i++) {
-            mx = fmaxf(mx, mxs[i][qi]);
-            bad |= bws[i][qi];
-        }
-        bad = bad || __builtin_isinf(mx);
-        const int64_t nv = n >= 8 ? (n & ~(int64_t)7) : 0;
-        if (!bad)
-            for (int64_t j = jj; j < n; j += JS) {
-                const float x = ew[j * QG + qi] - mx;
-                ew[j * QG + qi] = j < nv ? cephes_exp(x) : (float)exp((double)x);
-            }
-        if (t < QG) bads[t] = bad;
-    }
-    __syncthreads();
-    // 2. The sums: thread 8i + c (i < QG) runs query i's chain c.
-    if (t < 8 * QG) {
-        const int qi = t >> 3, c = t & 7;
-        const int64_t n = ns[qi], nv = n >= 8 ? (n & ~(int64_t)7) : 0;
-        float sl = 0.f;
-        for (int64_t j = c; j < nv; j += 8) sl = sl + ew[j * QG + qi];
-        const int g = lane & ~7;
-        float sum = ((__shfl(sl, g) + __shfl(sl, g + 4)) + (__shfl(sl, g + 1) + __shfl(sl, g + 5))) +
-                    ((__shfl(sl, g + 2) + __shfl(sl, g + 6)) + (__shfl(sl, g + 3) + __shfl(sl, g + 7)));
-        if (c == 0) {
-            for (int64_t j = nv; j < n; j++) sum = sum + ew[j * QG + qi];
-            sums[qi] = sum;
-        }
-    }
-    __syncthreads();
-    // 3. The chains of this wave's queries, in passes of the workgroup's
-    // queries that share the first entry. Keys below every live query's
-    // count run unmasked, whole value blocks at a time; the rest key by key
-    // with each query's own bound. Every bound is a scalar.
-    const int q0 = QW * qg;
-    float acc[QW];
-#pragma unroll
-    for (int i = 0; i < QW; i++) acc[i] = 0.f;
-    int64_t nq[QW];
-    int bq[QW];
-#pragma unroll
-    for (int i = 0; i < QW; i++) {
-        nq[i] = uni64(ns[q0 + i]);
-        bq[i] = __builtin_amdgcn_readfirstlane(bads[q0 + i]);
-    }
-    int first = -1;
-    bool same = true;
-    for (int i = 0; i < QG; i++) {
-        const int64_t ni = uni64(ns[i]);
-        if (ni <= 0) continue;
-        if (first < 0) first = i;
-        else same = same && uni64(k0s[i]) == uni64(k0s[first]);
-    }
-    const VT* vbase = (const VT*)vc;
-    for (int pass = 0; pass < (same ? 1 : QG); pass++) {
-        if (!same && (pass < q0 || pass >= q0 + QW)) continue;  // not this wave's query
-        const int src = same ? (first < 0 ? 0 : first) : pass;
-        if (uni64(ns[src]) <= 0) continue;
-        const int64_t k0 = uni64(k0s[src]);
-        uint32_t live = 0;
-        int64_t nmin = INT64_MAX, nmax = 0;
-#pragma unroll
-        for (int i = 0; i < QW; i++) {
-            const bool in = nq[i] > 0 && !bq[i] && (same || q0 + i == pass);
-            if (in) {
-                live |= 1u << i;
-                nmin = nq[i] < nmin ? nq[i] : nmin;
-                nmax = nq[i] > nmax ? nq[i] : nmax;
-            }
-        }
-        if (!live) continue;
-        const int64_t nfull = live == (1u << QW) - 1 ? nmin : 0;  // keys every query of the wave sees
-        const int64_t off = k0 & 7;                                 // key k0's place in its value block
-        const int64_t kbeg = k0 - off;
-        const int64_t nblk = (off + nmax + 7) >> 3;
-        auto vload = [&](int64_t ib, uint4& x0, uint4& x1) {
-            const VT* vp = vbase + vcache_at(hk, kbeg + 8 * (ib < nblk ? ib : nblk - 1), d, D, C);
-            x0 = *(const uint4*)vp;
-            x1 = x0;
-            if constexpr (!F16) x1 = *(const uint4*)(vp + 4);
-        };
-        constexpr int PF = 4;
-        uint4 c0[PF], c1[PF];
-#pragma unroll
-        for (int u = 0; u < PF; u++) vload(u, c0[u], c1[u]);
-        for (int64_t ib0 = 0; ib0 < nblk; ib0 += PF) {
-            uint4 n0[PF], n1[PF];
-#pragma unroll
-            for (int u = 0; u < PF; u++) vload(ib0 + PF + u, n0[u], n1[u]);
-#pragma unroll
-            for (int u = 0; u < PF; u++) {
-                const int64_t ib = ib0 + u;
-                if (ib >= nblk) break;
-                const int64_t j0 = 8 * ib - off;  // key index of the block's entry 0
-                if (j0 >= 0 && j0 + 8 <= nfull) {
-                    // a whole block every query sees: its weights first, then the fmas
-                    float4 ea[8], eb[8];
-#pragma unroll
-                    for (int kk = 0; kk < 8; kk++) {
-                        const float4* er = (const float4*)(ew + (j0 + kk) * QG + q0);
-                        ea[kk] = er[0];
-                        eb[kk] = er[1];
-                    }
-#pragma unroll
-                    for (int kk = 0; kk < 8; kk++) {
-                        const float v = att_vget<F16>(c0[u], c1[u], kk);
-                        const float e[8] = {ea[kk].x, ea[kk].y, ea[kk].z, ea[kk].w,
-                                            eb[kk].x, eb[kk].y, eb[kk].z, eb[kk].w};
-#pragma unroll
-                        for (int i = 0; i < QW; i++) acc[i] = __builtin_fmaf(e[i], v, acc[i]);
-                    }
-                } else {
-                    // the block's keys one at a time, each query to its own count
-#pragma unroll
-                    for (int kk = 0; kk < 8; kk++) {
-                        const int64_t j = j0 + kk;
-                        if (j < 0 || j >= nmax) continue;
-                        const float4* er = (const float4*)(ew + j * QG + q0);
-                        const float4 ea = er[0], eb = er[1];
-                        const float e[8] = {ea.x, ea.y, ea.z, ea.w, eb.x, eb.y, eb.z, eb.w};
-                        const float v = att_vget<F16>(c0[u], c1[u], kk);
-#pragma unroll
-                        for (int i = 0; i < QW; i++)
-                            if (((live >> i) & 1) && j < nq[i]) acc[i] = __builtin_fmaf(e[i], v, acc[i]);
-                    }
-                }
-            }
-#pragma unroll
-            for (int u = 0; u < PF; u++) {
-                c0[u] = n0[u];
-                c1[u] = n1[u];
-            }
-        }
-    }
-#pragma unroll
-    for (int i = 0; i < QW; i++) {
-        const int qi = q0 + i, tq = t0 + qi;
-        if (tq < T)
-            out[((int64_t)tq * H + h) * D + d] = ns[qi] <= 0 ? 0.f : (bads[qi] ? __builtin_nanf("") : acc[i] / sums[qi]);
-    }
-}
-
 template <bool F16, int QT>
 static void launch_att_scores(dim3 grid, const float* q, const void* kc, const int64_t* kend, const int64_t* kstart,
                               int T, int H, int Hkv, int D, int64_t C, int64_t maxk, float* ws, hipStream_t s) {
@@ -1632,31 +1277,16 @@ hipError_t launch_attention(const float* q, const void* kc, const void* vc, cons
                             int T, int H, int Hkv, int D, int64_t C, int64_t maxk, int f16, float* out, float* ws,
                             hipStream_t s) {
     if (D > 512 || D % 8 || H % Hkv || maxk < 1 || maxk > ATT_MAXC || T < 1) return hipErrorInvalidValue;
-    // many queries: four per workgroup, sharing the key and value loads
-    const bool many = T >= 16 && D % 64 == 0 && maxk <= 2048;
     const unsigned tiles = (unsigned)((maxk + 63) / 64);
-    // many queries, D = 64 or 128 (D = 128 with an f16 cache: the key in 64
-    // registers), up to 1024 keys: a key per lane for the scores and the
-    // queries' chains side by side for the weighted sum
-    // (measured on MI355X at the 8B heads: 125 against 224 us at 512 rows;
-    // slower below about 256 rows, whose grids are too small)
-    if (many && T >= 256 && (D == 64 || (D == 128 && f16)) && maxk <= 1024 && T <= 65535 &&
-        (((uintptr_t)q | (uintptr_t)kc | (uintptr_t)vc) & 15) == 0) {
-        const dim3 g1((unsigned)((maxk + 255) / 256), (unsigned)H, (unsigned)((T + ATT_KPL_QG - 1) / ATT_KPL_QG));
-        const dim3 g2(1, (unsigned)H, (unsigned)((T + ATT_QPL_QG - 1) / ATT_QPL_QG));
-        const size_t lds = (size_t)maxk * ATT_QPL_QG * 4;
-#define ATT_PROMPT(F, DD)                                                                                         \
-    hipLaunchKernelGGL((att_scores_kpl_kernel<F, DD>), g1, dim3(256), 0, s, q, kc, kend, kstart, T, H, Hkv, C, maxk, \
-                       ws);                                                                                       \
-    hipLaunchKernelGGL((att_wsum_qpl_kernel<F, DD>), g2, dim3(DD * ATT_QPL_QG / ATT_QPL_QW), lds, s, vc, kend,         \
-                       kstart, T, H, Hkv, C, maxk, ws,                                                           \
-                       out)
-        if (f16 && D == 128) { ATT_PROMPT(true, 128); }
-        else if (f16) { ATT_PROMPT(true, 64); }
-        else { ATT_PROMPT(false, 64); }
-#undef ATT_PROMPT
-        return hipGetLastError();
-    }
+    // from 16 queries at D = 64 or 128: the matrix cores (measured on MI355X
+    // at 32 heads, D = 128: 16 queries of 64 keys 16.7 -> 13.9 us, of 2048
+    // keys 32 -> 14). C below 2^30: its 32-bit key indices.
+    if (T >= 16 && (D == 64 || D == 128) && C < (1 << 30) &&
+        (((uintptr_t)q | (uintptr_t)kc | (uintptr_t)vc) & 15) == 0)
+        return launch_attention_mfma(q, kc, vc, kend, kstart, T, H, Hkv, D, C, maxk, f16, out, ws, s);
+    // many queries of other sizes: four per workgroup, sharing the key and
+    // value loads
+    const bool many = T >= 16 && D % 64 == 0 && maxk <= 2048;
     if (many) {
         const dim3 grid(tiles, (unsigned)H, (unsigned)((T + 3) / 4));
         if (f16) launch_att_scores<true, 4>(grid, q, kc, kend, kstart, T, H, Hkv, D, C, maxk, ws, s);

@@ -211,6 +211,10 @@ hipError_t launch_rope(float* x, const int64_t* pos, const double* inv_freq, int
                        int interleaved, hipStream_t s);
 hipError_t launch_kv_store(const float* k, const float* v, const int64_t* pos, int T, int Hkv, int D, int64_t C, void* kc,
                            void* vc, int f16, hipStream_t s);
+// D = 64 or 128, q, kc and vc 16-byte aligned (attention_mfma.hip).
+hipError_t launch_attention_mfma(const float* q, const void* kc, const void* vc, const int64_t* kend,
+                                 const int64_t* kstart, int T, int H, int Hkv, int D, int64_t C, int64_t maxk, int f16,
+                                 float* out, float* ws, hipStream_t s);
 hipError_t launch_attention(const float* q, const void* kc, const void* vc, const int64_t* kend, const int64_t* kstart,
                             int T, int H, int Hkv, int D, int64_t C, int64_t maxk, int f16, float* out, float* ws,
                             hipStream_t s);
