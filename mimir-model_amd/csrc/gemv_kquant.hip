@@ -108,8 +108,8 @@ __device__ __forceinline__ void quad_of(int pb, int nb, int& b, int& r0) {
 // weights: the load counter being in order, anything issued after the
 // weights would wait for all of them. Every load is unconditional (clamped
 // in bounds) in straight-line code, and every loaded pair is consumed.
-// SW (swiglu epilogue, M = 1, R = 2U): local rows 0..U-1 are gate rows
-// tile*U.., rows U..2U-1 the same rows of up; a quad of U rows is one
+// SW (swiglu epilogue, M = 1, RH = R / 2 a multiple of U): local rows
+// 0..RH-1 are gate rows tile*RH.., rows RH..R-1 the same rows of up; a quad of U rows is one
 // matrix's, so each quad loads from its matrix's tile base. The rows'
 // results meet in LDS and out[n] = swiglu(gate[n], up[n]) is written.
 // One workgroup's tile `tile` of the matrix A.W (A.wref, A.bias, A.y, A.N
@@ -118,11 +118,12 @@ template <uint32_t DT, int M, int R, bool SW, int U = PAIRS_U>
 __device__ __forceinline__ void pairs_tile(GemvArgs A, int tile, uint8_t* smem) {
     constexpr bool SHARED = R % U == 0;  // a group's U pairs share one block
     constexpr bool PRE = M == 1;         // activation loaded before the weights
-    static_assert(!SW || (M == 1 && R == 2 * U && SHARED), "swiglu epilogue: one row, a gate and an up quad");
+    constexpr int RH = R / 2;            // SW: rows of each matrix
+    static_assert(!SW || (M == 1 && RH % U == 0 && SHARED), "swiglu epilogue: one row, gate and up quads");
     const int g = threadIdx.x >> 3, l = threadIdx.x & 7, t = threadIdx.x;
-    const int nb = A.nb, row0 = tile * (SW ? U : R), npairs = R * nb;
+    const int nb = A.nb, row0 = tile * (SW ? RH : R), npairs = R * nb;
     // The tile's R rows: a 4-byte-aligned base (Q6_K rows are 2-byte
-    // aligned) and 32-bit offsets from it (SW: the U rows of each matrix).
+    // aligned) and 32-bit offsets from it (SW: the RH rows of each matrix).
     const int64_t tbyte = (int64_t)row0 * A.rb;
     const uint8_t* Wt = A.W + (tbyte & ~(int64_t)3);
     const uint32_t tadj = (uint32_t)(tbyte & 3), rb32 = (uint32_t)A.rb;
@@ -138,8 +139,8 @@ __device__ __forceinline__ void pairs_tile(GemvArgs A, int tile, uint8_t* smem) 
     int fm = min(t, R * M - 1) % M;
     asm volatile("v_mov_b32 %0, %1" : "=v"(fm) : "v"(fm));  // a vector index: ok[] through the vector cache
     const int fr = min(t, R * M - 1) / M;
-    const PairMat& FM = SW && fr >= U ? A.mat[1] : A.mat[0];
-    const int frow = SW ? row0 + (fr & (U - 1)) : min(row0 + fr, A.N - 1);
+    const PairMat& FM = SW && fr >= RH ? A.mat[1] : A.mat[0];
+    const int frow = SW ? row0 + (fr & (RH - 1)) : min(row0 + fr, A.N - 1);
     const int wr = SW ? FM.wref[frow] : A.wref[frow], okm = A.ok[fm];
     const float* fbias = SW ? FM.bias : A.bias;
     const float bias = fbias ? fbias[frow] : 0.f;
@@ -176,8 +177,8 @@ __device__ __forceinline__ void pairs_tile(GemvArgs A, int tile, uint8_t* smem) 
                 b = p / R;
                 r = min(p - b * R, rlast);
             }
-            const uint8_t* Wb = SW && r >= U ? Wt1 : Wt;
-            const uint32_t off = tadj + (uint32_t)(SW ? (r & (U - 1)) : r) * rb32 + (uint32_t)b * KQ<DT>::BYTES;
+            const uint8_t* Wb = SW && r >= RH ? Wt1 : Wt;
+            const uint32_t off = tadj + (uint32_t)(SW ? (r & (RH - 1)) : r) * rb32 + (uint32_t)b * KQ<DT>::BYTES;
             if constexpr (DT == DT_Q4_K) {
                 hdr[u] = *(const u32x4*)(Wb + off);
                 qv[u] = *(const u32x4*)(Wb + (off + 16 * l + 16));
@@ -239,7 +240,7 @@ __device__ __forceinline__ void pairs_tile(GemvArgs A, int tile, uint8_t* smem) 
     // The serial float chain, one lane per (weight row, activation row).
     float* yr = (float*)(refused + R * M);  // SW: [R] the rows' results
     if (t < R * M) {
-        const int r = t / M, m = t - r * M, row = SW ? row0 + (r & (U - 1)) : row0 + r;
+        const int r = t / M, m = t - r * M, row = SW ? row0 + (r & (RH - 1)) : row0 + r;
         if (row < A.N && !flag) {
             float tot = 0.f, off = 0.f;
             for (int b = 0; b < nb; b++) {
@@ -255,9 +256,9 @@ __device__ __forceinline__ void pairs_tile(GemvArgs A, int tile, uint8_t* smem) 
     }
     // The float32 path for refused pairs, one group of eight lanes per pair.
     for (int qq = g; qq < R * M; qq += 32) {
-        const int r = qq / M, m = qq - r * M, row = SW ? row0 + (r & (U - 1)) : row0 + r;
+        const int r = qq / M, m = qq - r * M, row = SW ? row0 + (r & (RH - 1)) : row0 + r;
         if (row < A.N && refused[qq]) {
-            const PairMat& RM = SW && r >= U ? A.mat[1] : A.mat[0];
+            const PairMat& RM = SW && r >= RH ? A.mat[1] : A.mat[0];
             const uint8_t* Wr = SW ? RM.W : A.W;
             const float* br = SW ? RM.bias : A.bias;
             float res = f32dot_g8<DT>(Wr + (int64_t)row * A.rb, A.x + (int64_t)m * A.K, A.K, A.fused != 0);
@@ -272,7 +273,7 @@ __device__ __forceinline__ void pairs_tile(GemvArgs A, int tile, uint8_t* smem) 
         // swiglu.v1 of (gate, up) row n: the reference's SiluMulF32 on its pieces
         __syncthreads();
         const int n = row0 + t;
-        if (t < U && n < A.N) A.sw[n] = swiglu_at(yr[t], yr[t + U], n, A.sw_total, A.sw_chunk);
+        if (t < RH && n < A.N) A.sw[n] = swiglu_at(yr[t], yr[t + RH], n, A.sw_total, A.sw_chunk);
     }
 }
 
@@ -294,13 +295,21 @@ __global__ __launch_bounds__(256) void gemv_a8k_pairs_kernel(GemvArgs A) {
 }
 
 // gate and up at one row with swiglu in the epilogue (Q4_K, N % U == 0).
-static hipError_t launch_pairs_swiglu(GemvArgs A, hipStream_t stream) {
-    constexpr int U = PAIRS_U, R = 2 * U;
+template <int R>
+static hipError_t launch_pairs_swiglu_r(GemvArgs A, hipStream_t stream) {
     A.mat[0].tile0 = A.mat[1].tile0 = 0;
-    const int tiles = A.N / U;
+    const int tiles = A.N / (R / 2);
     const size_t lds = (size_t)R * A.nb * 16 + (size_t)R * 4 + (size_t)R * 4;
     hipLaunchKernelGGL((gemv_a8k_pairs_kernel<DT_Q4_K, 1, R, true>), dim3((unsigned)tiles), dim3(256), lds, stream, A);
     return hipGetLastError();
+}
+// Twice the rows where these would fill at most half of a pass's pairs (K up
+// to 2048) and 512 workgroups are left (measured on MI355X: the whole step at
+// 2048 x 8192 20.3 -> 18.6 us together with down's rows).
+static hipError_t launch_pairs_swiglu(const GemvArgs& A, hipStream_t stream) {
+    constexpr int R = 2 * PAIRS_U;
+    if (A.nb * R <= 16 * PAIRS_U && A.N % R == 0 && A.N / R >= 512) return launch_pairs_swiglu_r<2 * R>(A, stream);
+    return launch_pairs_swiglu_r<R>(A, stream);
 }
 
 template <uint32_t DT, int M, int R, int U = PAIRS_U>
@@ -315,11 +324,26 @@ static hipError_t launch_pairs_r(GemvArgs A, hipStream_t stream) {
     return hipGetLastError();
 }
 
-// Rows per workgroup: enough (row, block) pairs to keep 32 groups busy, as
-// many workgroups as possible, and the pair table within 48 KB of LDS.
+// Rows per workgroup. A pass of the workgroup takes 32 U pairs and what is
+// left of the last one idles, so for one activation row, from the rows that
+// give 1024 workgroups (up to 8), more rows (up to 32) are taken where the
+// pairs then need fewer passes a row and fill at least half a pass, with 512
+// workgroups left up to 8 rows, 1024 above, 1536 for several passes (measured
+// on MI355X, us: Q6_K 128256 x 2048 64.3 -> 41.4 with 16 rows, 32768 x 5120
+// 41.0 -> 36.4, 2048 x 8192 10.4 -> 8.4 with 4 rows; but 5120 x 5120, as many
+// passes a row with half the workgroups, 8.2 -> 9.2, and 40000 x 2816, three
+// passes and 1250 workgroups, 14.3 -> 14.6). The pair table stays within 48 KB
+// of LDS.
 static int pairs_rows(int N, int nb, int M) {
+    auto fits = [&](int r, int tiles) { return (N + r - 1) / r >= tiles && (size_t)r * nb * M * 16 <= 48 * 1024; };
+    auto passes = [&](int r) { return (r * nb + 32 * PAIRS_U - 1) / (32 * PAIRS_U); };
     int R = 8;
-    while (R > 1 && ((N + R - 1) / R < 1024 || (size_t)R * nb * M * 16 > 48 * 1024)) R >>= 1;
+    while (R > 1 && !fits(R, 1024)) R >>= 1;
+    if (M > 1) return R;
+    for (int r = 2 * R; r <= 32; r *= 2)
+        if (fits(r, passes(r) > 1 ? 1536 : (r > 8 ? 1024 : 512)) && 2 * r * nb >= 32 * PAIRS_U &&
+            r * passes(R) > R * passes(r))
+            R = r;
     return R;
 }
 
@@ -328,7 +352,12 @@ static hipError_t launch_pairs(GemvArgs A, hipStream_t stream) {
     int total_n = 0;
     for (int i = 0; i < A.nmat; i++) total_n += A.mat[i].N;
 
-    switch (pairs_rows(total_n, A.nb, M)) {
+    const int R = pairs_rows(total_n, A.nb, M);
+    if constexpr (M == 1) {
+        if (R == 32) return launch_pairs_r<DT, M, 32>(A, stream);
+        if (R == 16) return launch_pairs_r<DT, M, 16>(A, stream);
+    }
+    switch (R) {
     case 8: return launch_pairs_r<DT, M, 8>(A, stream);
     case 4: return launch_pairs_r<DT, M, 4>(A, stream);
     case 2: return launch_pairs_r<DT, M, 2>(A, stream);
