@@ -67,6 +67,7 @@ compared with the GPU's (8 tokens; the 8B shape on a 32-token prompt).
 import argparse
 import ctypes
 import json
+import math
 import os
 import platform
 import sys
@@ -351,7 +352,7 @@ def main():
                          "products as one chain launch (mimg_linear_a8_chain_dev, one row only)")
     ap.add_argument("--graph-steps", type=int, default=0,
                     help="steps captured in one HIP graph (consecutive rotation layers; divides --rotate; "
-                         "default: --rotate)")
+                         "default: the largest that divides --rotate, --steps and --warmup)")
     ap.add_argument("--roofline-replays", type=int, default=8,
                     help="replays of the graph of --rotate single-kernel launches timed for the roofline")
     args = ap.parse_args()
@@ -500,10 +501,10 @@ def main():
                                          [yd[c[0]].ptr for c in grp], ws[i].ptr, ws_bytes[i], stream.handle)
 
     # A graph holds gs consecutive steps (layers l .. l+gs-1 of the rotation:
-    # by default all 32, one token's linear sets, as a decode step's graph
-    # holds all of a token's layers); with gs = 1 the host launches one graph
-    # per step.
-    gs = args.graph_steps or args.rotate
+    # all 32 at the default --steps and --warmup, one token's linear sets, as a
+    # decode step's graph holds all of a token's layers); with gs = 1 the host
+    # launches one graph per step.
+    gs = args.graph_steps or math.gcd(args.rotate, args.steps, args.warmup)
     if args.rotate % gs or args.steps % gs or args.warmup % gs:
         raise SystemExit("--graph-steps must divide --rotate, --steps and --warmup")
     if args.eager:
