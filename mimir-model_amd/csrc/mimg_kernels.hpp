@@ -215,6 +215,10 @@ hipError_t launch_kv_store(const float* k, const float* v, const int64_t* pos, i
 hipError_t launch_attention_mfma(const float* q, const void* kc, const void* vc, const int64_t* kend,
                                  const int64_t* kstart, int T, int H, int Hkv, int D, int64_t C, int64_t maxk, int f16,
                                  float* out, float* ws, hipStream_t s);
+// The scores alone, few queries: at most 8 query heads a kv head, D = 64 or
+// 128, q and kc 16-byte aligned.
+hipError_t launch_att_scores_mfma(const float* q, const void* kc, const int64_t* kend, const int64_t* kstart, int T, int H,
+                                  int Hkv, int D, int64_t C, int64_t maxk, int f16, float* ws, hipStream_t s);
 hipError_t launch_attention(const float* q, const void* kc, const void* vc, const int64_t* kend, const int64_t* kstart,
                             int T, int H, int Hkv, int D, int64_t C, int64_t maxk, int f16, float* out, float* ws,
                             hipStream_t s);

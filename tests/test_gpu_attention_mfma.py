@@ -1,4 +1,5 @@
-"""Attention from 16 query rows on the matrix cores (attention_mfma.hip)
+"""Attention on the matrix cores (attention_mfma.hip; all of it from 16 query
+rows, the scores below)
 against the C restatement of the reference's attendRow, bit for bit: query
 heads per kv head that do and do not divide the row tiles, both sum tiles
 (4 and 16 rows a wave), ragged last tiles, sequences that start inside a value
@@ -55,6 +56,26 @@ def test_rows_and_tiles(gpu, oracle, f16, T, H, Hkv, D, slots, C):
         got = _call(gpu, q, kc, vc, gend, None, C)
     else:
         got = _call(gpu, q, kc, vc, gend, start, C)
+    assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), np.argwhere(got != want)[:5]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("f16", [False, True], ids=["f32cache", "f16cache"])
+@pytest.mark.parametrize("T,H,Hkv,D,C", [(4, 16, 8, 64, 520), (3, 24, 8, 128, 705), (9, 10, 2, 64, 961),
+                                         (8, 64, 8, 128, 321), (2, 14, 2, 128, 4100), (1, 32, 8, 64, 2049)])
+def test_decode_scores(gpu, oracle, f16, T, H, Hkv, D, C):
+    """Decode batches, a sequence a row: 2 to 8 query heads a kv head, every
+    count of keys mod 4, the last tile of one key and full."""
+    rng = np.random.default_rng(T * 10 + H + C)
+    kc = rng.standard_normal((Hkv, T * C, D)).astype(np.float16 if f16 else np.float32)
+    vc = rng.standard_normal((Hkv, T * C, D)).astype(kc.dtype)
+    q = rng.standard_normal((T, H, D)).astype(np.float32)
+    start = (np.arange(T) * C).astype(np.int64)
+    end = start + C - 1 - np.array([t if t < 6 else 64 * t for t in range(T)])
+    for t in range(T):
+        kc[:, end[t] + 1:(t + 1) * C], vc[:, end[t] + 1:(t + 1) * C] = np.nan, np.inf
+    got = _call(gpu, q, kc, vc, end, start, C)
+    want = oracle.attention(q, kc, vc, end, start, threads=8)
     assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), np.argwhere(got != want)[:5]
 
 
