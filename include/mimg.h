@@ -367,8 +367,8 @@ int mimg_matmul_a8_quantized_q8_0_tiled_dev(uint64_t w, const float *x, int64_t 
  * block j (Q6_K: both sub-blocks of 16 with their scales), tot = fma(d, t,
  * tot); Q4_K also off = fma(dmin * f32(m_j), dbs_j, off); result tot - off
  * (Q4_K) or tot, plus the bias. Each weight byte is read once per tile of
- * activation rows (the lane-order GEMV of the other entry points reads it
- * once per eight rows). A tolerance claim as the Q8_0 form: within the
+ * activation rows (the lane-order K-quant GEMV of the other entry points reads
+ * it once per eight rows). A tolerance claim as the Q8_0 form: within the
  * spec's dequant_matmul_a8 bound (spec/stdlib.md:260-275); each row's result
  * depends on that row alone; refused rows take the reference-order float32
  * path. Returns MIMG_NOT_HANDLED for shapes or weight alignments it does

@@ -1,9 +1,8 @@
 // Prefill GEMM for small grids: Q4_K / Q6_K weights x 8-bit activations in
 // blocks of 256 on v_mfma_i32_16x16x64_i8, 64 weight rows x 128 activation
-// rows per workgroup of eight waves. gemm_kquant.hip's 32 x 32 x 32 kernel
-// takes 128 x 128 tiles; where that gives fewer workgroups than the GPU has
-// CUs (few weight rows or few activation rows, e.g. 64 prompt rows) this one
-// runs instead. Same result, bit for bit (both equal the decode GEMV):
+// rows per workgroup of eight waves. The 32 x 32 x 32 kernels take larger tiles
+// (gemm_kquant.hip: Q6_K, gemm_q4k.hip: Q4_K); where those give too few
+// workgroups (few weight rows or few activation rows) this one runs instead. Same result, bit for bit (both equal the decode GEMV):
 // per (weight row n, activation row m) and block b the exact int32
 //   Q4_K  S = sum_k sc_s(k) q_k y_k,   M = sum_k m_s(k) y_k (= sum_s m_s xs_s)
 //   Q6_K  S = sum_k sc_s(k) (q_k - 32) y_k

@@ -7,7 +7,7 @@
 //
 // Numerics: the same exact int32 block sums as the pair kernel and the GEMM
 // (reference internal/kernels/q8k.go dotQ8KRef, q8k_test.go:38-102; the
-// GEMM's split of the scaled weights into two int8 planes, gemm_kquant.hip),
+// GEMM's split of the scaled weights into two int8 planes, gemm_q4k.hip),
 // then per (weight row, activation row) the serial chain
 // tot = fma(f32(S_b), d_b*dx_b, tot) (and off for Q4_K's mins) in block
 // order: bit for bit the one-row kernel.
