@@ -30,6 +30,16 @@
 // the other rows' sums. Rows with different first keys (several sequences)
 // run one first key at a time.
 //
+// EACH, for calls whose sequences may have few rows each (decode batches of
+// many sequences, few query heads a kv head): a 32-row tile of scores and a
+// pass over a first key would mostly work for rows that don't see the keys. A
+// scores wave whose keys at most eight rows see takes those rows, four at a
+// time, on the 4x4x1_16b (an eighth of the matrix time, the same operands);
+// wsum has workgroups of four rows, one per first key of the four, which skip
+// the weights of rows of other passes. A prompt's waves take the 32-row tile
+// as before. These are instances of their own: the branches in the others'
+// code cost a prompt 3 to 10 %.
+//
 // Bound: the matrix cores' f32 rate (measured 18 ns a 16x16x1_4b and 32 ns a
 // 32x32x1_2b, 2x the vector unit's fmas) and, in wsum, a wave's serial chain
 // over the keys (6.9 ns a key with RT = 4, 18 with 16); below a few hundred
@@ -37,8 +47,8 @@
 // Measured on MI355X, us, against a key a lane for the scores and eight chains
 // a lane for the sum on the vector unit (32 heads, 8 kv heads, D = 128, f16):
 // 512 rows 125 -> 56 (scores 65 -> 24, sum 63 -> 32), 2000 rows 3197 -> 510,
-// 64 rows 37.7 -> 14.9, 16 rows 16.7 -> 13.9; 32 sequences of 700 keys, a row
-// each, 128 -> 60. Loading the next tile's keys ahead in scores_kernel cost a
+// 64 rows 37.7 -> 14.9, 16 rows 16.7 -> 13.9; D = 64: 512 rows 93 -> 62 (f16),
+// 94 -> 70 (f32). Loading the next tile's keys ahead in scores_kernel cost a
 // wave a SIMD and measured 61 us at 512 rows.
 #include <type_traits>
 
@@ -89,7 +99,7 @@ __device__ __forceinline__ Row row_of(const Args& A, int hk, uint32_t rho) {
 
 constexpr int SROWS = 32, SKEYS = 128;
 
-template <bool F16, int D>
+template <bool F16, int D, bool EACH>
 __global__ __launch_bounds__(256, 2) void scores_kernel(Args A) {
     constexpr int DM = D / 8, QS = D + 4;  // a row in LDS, padded by four banks
     __shared__ __align__(16) float qs[SROWS * QS];
@@ -120,7 +130,9 @@ __global__ __launch_bounds__(256, 2) void scores_kernel(Args A) {
     const float scale = (float)(1.0 / sqrt((double)D));
     for (int kt = kt0; kt < kfin; kt += SKEYS * (int)gridDim.y) {
         const int kb = kt + 32 * w;  // this wave's first key
-        if (!__any(r.n > 0 && r.k0 < kb + 32 && r.k0 + r.n > kb)) continue;
+        // the rows that see any of its keys
+        uint32_t seen = (uint32_t)__ballot(r.n > 0 && r.k0 < kb + 32 && r.k0 + r.n > kb);
+        if (seen == 0) continue;
         const int a = kb + a32;
         const int64_t ac = a < A.C ? a : A.C - 1;  // past the cache: its last key, unstored
         using KT = typename std::conditional<F16, uint2, float4>::type;
@@ -128,13 +140,7 @@ __global__ __launch_bounds__(256, 2) void scores_kernel(Args A) {
         const uint8_t* kp = (const uint8_t*)A.kc + (((int64_t)hk * A.C + ac) * D + 4 * g) * (F16 ? 2 : 4);
 #pragma unroll
         for (int m = 0; m < DM; m++) kw[m] = *(const KT*)(kp + m * (F16 ? 16 : 32));
-        const float* qr = qs + a32 * QS + 4 * g;
-        v32f acc[4];
-#pragma unroll
-        for (int m = 0; m < DM; m++) {
-            const float4 q4 = *(const float4*)(qr + 8 * m);
-            const float qv[4] = {q4.x, q4.y, q4.z, q4.w};
-            float kv[4];
+        auto key4 = [&](int m, float (&kv)[4]) {
             if constexpr (F16) {
                 const uint32_t wd[2] = {kw[m].x, kw[m].y};
 #pragma unroll
@@ -143,6 +149,56 @@ __global__ __launch_bounds__(256, 2) void scores_kernel(Args A) {
             } else {
                 kv[0] = kw[m].x, kv[1] = kw[m].y, kv[2] = kw[m].z, kv[3] = kw[m].w;
             }
+        };
+        if (EACH && __popc(seen) <= 8) {
+            // four rows a turn on the 4x4x1_16b: lane l gives the (l % 4)th
+            // row's q and gets all four's chains 4 g + i against its own key
+            while (seen) {
+                int sel[4], nsel = 0;
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    sel[i] = seen ? __builtin_ctz(seen) : sel[i > 0 ? i - 1 : 0];
+                    nsel += seen != 0;
+                    seen &= seen - 1;
+                }
+                const float* qr = qs + (l & 2 ? (l & 1 ? sel[3] : sel[2]) : (l & 1 ? sel[1] : sel[0])) * QS + 4 * g;
+                v4f acc[4];
+#pragma unroll
+                for (int m = 0; m < DM; m++) {
+                    const float4 q4 = *(const float4*)(qr + 8 * m);
+                    const float qv[4] = {q4.x, q4.y, q4.z, q4.w};
+                    float kv[4];
+                    key4(m, kv);
+                    const v4f z = {};
+#pragma unroll
+                    for (int i = 0; i < 4; i++) acc[i] = __builtin_amdgcn_mfma_f32_4x4x1f32(qv[i], kv[i], m ? acc[i] : z, 0, 0, 0);
+                }
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    if (i >= nsel) break;
+                    const int4 ri = rinfo[sel[i]];
+                    const int j = a - ri.x, n = ri.y, n4 = n & ~3;
+                    const float h = (acc[0][i] + acc[1][i]) + (acc[2][i] + acc[3][i]);
+                    float p = h + lane_xor_f32<32>(h);
+                    if (__any(j >= n4)) {
+                        const float e0 = acc[0][i] + lane_xor_f32<32>(acc[0][i]), e1 = acc[1][i] + lane_xor_f32<32>(acc[1][i]);
+                        const float e2 = acc[2][i] + lane_xor_f32<32>(acc[2][i]), e3 = acc[3][i] + lane_xor_f32<32>(acc[3][i]);
+                        p = j >= n4 ? (e0 + e1) + (e2 + e3) : p;
+                    }
+                    if (g == 0 && j >= 0 && j < n)
+                        A.ws[(int64_t)(((uint64_t)(uint32_t)ri.w << 32) | (uint32_t)ri.z) + j] = p * scale;
+                }
+            }
+            continue;
+        }
+        const float* qr = qs + a32 * QS + 4 * g;
+        v32f acc[4];
+#pragma unroll
+        for (int m = 0; m < DM; m++) {
+            const float4 q4 = *(const float4*)(qr + 8 * m);
+            const float qv[4] = {q4.x, q4.y, q4.z, q4.w};
+            float kv[4];
+            key4(m, kv);
             const v32f z = {};
 #pragma unroll
             for (int i = 0; i < 4; i++) acc[i] = __builtin_amdgcn_mfma_f32_32x32x1f32(qv[i], kv[i], m ? acc[i] : z, 0, 0, 0);
@@ -185,10 +241,10 @@ struct Tile<4> {
     static __device__ __forceinline__ int dim(int, int l) { return l; }
 };
 
-template <bool F16, int D, int RT>
-__global__ __launch_bounds__(2 * D, 2) void wsum_kernel(Args A) {
+template <bool F16, int D, int RT, bool EACH>
+__global__ __launch_bounds__((EACH ? 1 : 2) * D, 2) void wsum_kernel(Args A) {
     using TL = Tile<RT>;
-    constexpr int R = 2 * RT, DH = D / 64, NT = 2 * D, NW = NT / 64;
+    constexpr int RG = EACH ? 1 : 2, R = RG * RT, DH = D / 64, NT = RG * D, NW = NT / 64;
     // keys of a chunk (64 for RT = 16: 128 measured the same with 30 more
     // registers); a row's weights in LDS, padded by four banks
     constexpr int KC = RT == 16 ? 64 : D, ES = KC + 4;
@@ -216,18 +272,19 @@ __global__ __launch_bounds__(2 * D, 2) void wsum_kernel(Args A) {
 
     uint64_t live = __ballot(r.n > 0);
     // rows that see no key: zeros
-    if (~live & ((1ull << R) - 1)) {
+    if ((!EACH || blockIdx.y == 0) && (~live & ((1ull << R) - 1))) {
         lds_barrier();
         for (int i = t; i < R * D; i += NT) {
             const int row = i / D;
             if (!((live >> row) & 1) && rho0 + row < rows) A.out[(int64_t)rhead[row] * D + i % D] = 0.f;
         }
     }
-    while (live) {
+    for (uint32_t pass = 0; live; pass++) {
         // the rows that share the first live row's first key
         const int k0 = __builtin_amdgcn_readlane(r.k0, __builtin_ctzll(live));
         const uint64_t in = __ballot(r.n > 0 && r.k0 == k0);
         live &= ~in;
+        if (EACH && pass % gridDim.y != blockIdx.y) continue;  // another workgroup's
         const bool mine = (in >> l) & 1;
         const int nl = mine ? r.n : 0;
         const int nall = wave_max_i32(nl);
@@ -328,13 +385,22 @@ __global__ __launch_bounds__(2 * D, 2) void wsum_kernel(Args A) {
         auto exps = [&](int ch) {
             float* eb = ew[ch & 1] + t % KC;
             const int j = KC * ch + us;
-#pragma unroll
-            for (int u = 0; u < EPT; u++) {
+            auto one = [&](int u) {
                 const int row = (t + NT * u) / KC, nv = un[u] & ~7;
                 const float e = cephes_exp(sv[u] - um[u]), et = tail[row][j & 7];
                 eb[row * ES] = (uint32_t)j < (uint32_t)nv ? e : ((uint32_t)j < (uint32_t)un[u] ? et : 0.f);
-                if (u % 4 == 3) __builtin_amdgcn_sched_barrier(0);  // four exps at a time: registers
+            };
+            if (!EACH || in == (1ull << R) - 1) {
+#pragma unroll
+                for (int u = 0; u < EPT; u++) {
+                    one(u);
+                    if (u % 4 == 3) __builtin_amdgcn_sched_barrier(0);  // four exps at a time: registers
+                }
+                return;
             }
+#pragma unroll
+            for (int u = 0; u < EPT; u++)
+                if (un[u] > 0) one(u);  // rows of other passes: what LDS holds, for sums that are dropped
         };
         float sl[SPT];
 #pragma unroll
@@ -544,12 +610,29 @@ static hipError_t launch(const Args& A, hipStream_t s) {
     // walked by as many workgroups as give about four a CU
     const int64_t kt = ((A.kstart ? A.C : A.maxk) + SKEYS - 1) / SKEYS, yt = 1024 / xt;
     const dim3 g1((unsigned)xt, (unsigned)(yt < 1 ? 1 : (yt < kt ? yt : kt)));
-    hipLaunchKernelGGL((scores_kernel<F16, D>), g1, dim3(256), 0, s, A);
+    // Up to four rows (query, head) a sequence on average (the cache holds
+    // C / maxk sequences): EACH. Measured on MI355X, f16, us, with it / without /
+    // on the vector unit, a query a sequence: 32 heads of 32 kv heads, D = 128,
+    // 16 sequences of 700 keys 52 / 175 / 112, 64 of 700 176 / 305 / 213, 128 of
+    // 64 58 / 85 / 46; D = 64, 64 of 700 92 / 267 / 158; 16 kv heads 95 / 167 /
+    // 181 (64 of 700); 8 kv heads 58 / 78 / 160; 4 kv heads (eight rows a
+    // sequence) 53 / 47 / 158. Two queries a sequence of 700 keys, 64 sequences,
+    // D = 64, 32 kv heads 98 / 211 / 175, 16 61 / 107 / 162; four queries, 16
+    // sequences, 32 kv heads 43 / 71 / 68, 16 (eight rows) 41 / 39 / 69. A prompt
+    // of 64 rows in a cache of 64 sequences 16.8 / 16.1 / 32.5.
+    if (A.kstart && A.G <= 4 && (int64_t)A.T * A.G * A.maxk <= 4 * A.C) {
+        hipLaunchKernelGGL((scores_kernel<F16, D, true>), g1, dim3(256), 0, s, A);
+        // four rows are of at most (G + 2) / G + 1 queries, each with its first key
+        const dim3 g2((unsigned)((rows + 3) / 4 * A.Hkv), (unsigned)((A.G + 2) / A.G + 1));
+        hipLaunchKernelGGL((wsum_kernel<F16, D, 4, true>), g2, dim3(D), 0, s, A);
+        return hipGetLastError();
+    }
+    hipLaunchKernelGGL((scores_kernel<F16, D, false>), g1, dim3(256), 0, s, A);
     // 16 rows a wave where that gives every CU a workgroup, else four (a
     // quarter of the rows a workgroup, and a key of the chain in 6.9 ns, not 18)
     const int64_t wt = (rows + 31) / 32 * A.Hkv;
-    if (wt >= 256) hipLaunchKernelGGL((wsum_kernel<F16, D, 16>), dim3((unsigned)wt), dim3(2 * D), 0, s, A);
-    else hipLaunchKernelGGL((wsum_kernel<F16, D, 4>), dim3((unsigned)((rows + 7) / 8 * A.Hkv)), dim3(2 * D), 0, s, A);
+    if (wt >= 256) hipLaunchKernelGGL((wsum_kernel<F16, D, 16, false>), dim3((unsigned)wt), dim3(2 * D), 0, s, A);
+    else hipLaunchKernelGGL((wsum_kernel<F16, D, 4, false>), dim3((unsigned)((rows + 7) / 8 * A.Hkv)), dim3(2 * D), 0, s, A);
     return hipGetLastError();
 }
 

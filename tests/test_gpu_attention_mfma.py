@@ -5,22 +5,24 @@ heads per kv head that do and do not divide the row tiles, both sum tiles
 (4 and 16 rows a wave), ragged last tiles, sequences that start inside a value
 block, rows that see no key, a row clipped to max_keys, and infinities and NaN
 in every cache entry that no row of the call may use. The addresses are
-checked on the CPU over adversarial ranges."""
+checked on the CPU over adversarial ranges in test_attention_bounds.py."""
 import numpy as np
 import pytest
 
 
-def _call(gpu, q, kc, vc, kend, kstart, maxk):
+def _call(gpu, q, kc, vc, kend, kstart, maxk, shift=0):
+    """shift: floats from a 16-byte boundary to q."""
     import hiprt as rt
 
     T, H, D = q.shape
     Hkv, C, _ = kc.shape
     bufs = [rt.DeviceBuffer.from_array(np.ascontiguousarray(a))
-            for a in (q, kc, gpu.pack_vcache(vc), kend, kstart if kstart is not None else kend)]
+            for a in (np.concatenate([np.zeros(shift, np.float32), q.ravel()]), kc, gpu.pack_vcache(vc), kend,
+                      kstart if kstart is not None else kend)]
     out = rt.DeviceBuffer.from_array(np.full(q.shape, 7, np.float32))
     wsb = gpu.attention_workspace_bytes(T, H, maxk)
     ws, s = rt.DeviceBuffer(wsb), rt.Stream()
-    gpu.attention_dev(bufs[0].ptr, bufs[1].ptr, bufs[2].ptr, bufs[3].ptr, bufs[4].ptr if kstart is not None else None,
+    gpu.attention_dev(bufs[0].ptr + 4 * shift, bufs[1].ptr, bufs[2].ptr, bufs[3].ptr, bufs[4].ptr if kstart is not None else None,
                       T, H, Hkv, D, C, maxk, kc.dtype == np.float16, out.ptr, ws.ptr, wsb, s.handle)
     s.sync()
     return out.download(np.float32).reshape(q.shape)
@@ -31,7 +33,9 @@ def _call(gpu, q, kc, vc, kend, kstart, maxk):
 @pytest.mark.parametrize("T,H,Hkv,D,slots,C", [(16, 4, 4, 64, 1, 40), (17, 6, 2, 128, 1, 130), (33, 8, 1, 64, 1, 300),
                                                (40, 12, 4, 128, 3, 77), (257, 32, 8, 128, 1, 261),
                                                (65, 64, 64, 64, 2, 129), (300, 10, 10, 128, 5, 90),
-                                               (23, 14, 2, 64, 2, 1030)])
+                                               (23, 14, 2, 64, 2, 1030), (257, 32, 8, 64, 1, 300),
+                                               (300, 32, 8, 128, 7, 61), (300, 32, 8, 64, 150, 13),
+                                               (21, 6, 3, 192, 2, 90), (40, 4, 1, 256, 3, 77)])
 def test_rows_and_tiles(gpu, oracle, f16, T, H, Hkv, D, slots, C):
     rng = np.random.default_rng(T * 10 + H + C)
     L = slots * C
@@ -80,6 +84,64 @@ def test_decode_scores(gpu, oracle, f16, T, H, Hkv, D, C):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("f16", [False, True], ids=["f32cache", "f16cache"])
+@pytest.mark.parametrize("T,H,Hkv,D,slots,L", [(16, 4, 4, 64, 16, 61), (33, 6, 2, 128, 40, 83), (64, 8, 8, 128, 64, 29),
+                                               (40, 8, 2, 64, 40, 300), (50, 4, 2, 128, 25, 131), (90, 3, 3, 64, 23, 17),
+                                               (19, 1, 1, 128, 5, 700), (70, 2, 2, 128, 70, 7)])
+def test_few_rows_a_sequence(gpu, oracle, f16, T, H, Hkv, D, slots, L):
+    """Up to four (query, head) rows a sequence on average: 1 to 4 query heads a
+    kv head, sequences that start inside value blocks, several queries of one
+    sequence, waves of 32 keys that several sequences share, rows without a key."""
+    rng = np.random.default_rng(T + D)
+    kc = rng.standard_normal((Hkv, slots * L, D)).astype(np.float16 if f16 else np.float32)
+    vc = rng.standard_normal((Hkv, slots * L, D)).astype(kc.dtype)
+    q = rng.standard_normal((T, H, D)).astype(np.float32)
+    start = (np.arange(T) * slots // T * L).astype(np.int64)
+    end = start + rng.integers(0, L - 1, T)  # every sequence's last entry unused
+    end[0], end[T - 1] = start[0], start[T - 1] + L - 2
+    used = np.zeros(slots * L, bool)
+    for t in range(T):
+        used[start[t]:end[t] + 1] = True
+    kc[:, ~used], vc[:, ~used] = np.nan, np.inf
+    want = oracle.attention(q, kc, vc, end, start, threads=8)
+    end[T // 3] = start[T // 3] - 1
+    want[T // 3] = 0
+    got = _call(gpu, q, kc, vc, end, start, L)
+    assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), np.argwhere(got != want)[:5]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,slots,L,D", [(40, 40, 64, 128), (9 * 4, 36, 50, 64)])
+def test_prompt_among_many_sequences(gpu, oracle, T, slots, L, D):
+    """One sequence's rows in a cache of as many sequences as there are rows:
+    waves of both kinds (few and many rows) in one call."""
+    H, Hkv = 4, 4
+    rng = np.random.default_rng(T)
+    kc, vc = (rng.standard_normal((Hkv, slots * L, D)).astype(np.float16) for _ in range(2))
+    q = rng.standard_normal((T, H, D)).astype(np.float32)
+    start = np.full(T, 3 * L, np.int64)
+    start[::9] = 5 * L + 1
+    end = start + np.minimum(np.arange(T), L - 2)
+    got = _call(gpu, q, kc, vc, end, start, L)
+    want = oracle.attention(q, kc, vc, end, start, threads=8)
+    assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), np.argwhere(got != want)[:5]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,D,f16", [(20, 128, True), (17, 64, False)])
+def test_unaligned_q(gpu, oracle, T, D, f16):
+    """q four bytes past a 16-byte boundary: the vector kernels, same bits."""
+    H, Hkv, C = 8, 4, 150
+    rng = np.random.default_rng(T)
+    kc, vc = (rng.standard_normal((Hkv, C, D)).astype(np.float16 if f16 else np.float32) for _ in range(2))
+    q = rng.standard_normal((T, H, D)).astype(np.float32)
+    end = (np.arange(T) * 5 + 3).astype(np.int64)
+    got = _call(gpu, q, kc, vc, end, None, C, shift=1)
+    want = oracle.attention(q, kc, vc, end, None, threads=8)
+    assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), np.argwhere(got != want)[:5]
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("T,maxk", [(20, 50), (300, 257)])
 def test_max_keys_and_nonfinite(gpu, oracle, T, maxk):
     """Rows past max_keys see their first max_keys keys; a NaN key gives NaN
@@ -95,42 +157,3 @@ def test_max_keys_and_nonfinite(gpu, oracle, T, maxk):
     assert np.array_equal(np.isnan(got), np.isnan(want))
     fin = ~np.isnan(want)
     assert np.array_equal(got[fin].view(np.uint32), want[fin].view(np.uint32))
-
-
-def _ranges(T, C, maxk, slots, rng):
-    start = rng.integers(0, slots, T) * (C // slots)
-    end = start + rng.integers(-1, max(C // slots, 1), T)
-    for t, (e, s) in enumerate([(-5, -1), (C + 9, C + 3), (C - 1, C - 1), (C * 2, -7), (maxk + 50, 0)]):
-        end[t], start[t] = e, s
-    k0 = np.clip(start, 0, C - 1)
-    return k0, np.clip(np.minimum(np.minimum(end + 1 - k0, C - k0), maxk), 0, None)
-
-
-@pytest.mark.parametrize("D,f16", [(64, True), (64, False), (128, True), (128, False)])
-@pytest.mark.parametrize("T,H,Hkv,C,maxk,slots", [(16, 4, 4, 7, 8192, 1), (37, 6, 2, 301, 100, 3), (65, 8, 1, 8200, 8192, 2),
-                                                  (257, 8, 8, 130, 130, 4)])
-def test_addresses_in_bounds(D, f16, T, H, Hkv, C, maxk, slots):
-    G, rows = H // Hkv, T * (H // Hkv)
-    k0, n = _ranges(T, C, maxk, slots, np.random.default_rng(T + C))
-    head = lambda hk, rho: min(rho, rows - 1) // G * H + hk * G + min(rho, rows - 1) % G
-    vblocks = (C + 7) // 8
-    for hk in {0, Hkv - 1}:
-        # scores_kernel: 32 rows, tiles of 128 keys, keys clamped to the cache
-        for rho0 in range(0, rows, 32):
-            ts = [r // G for r in range(rho0, min(rho0 + 32, rows)) if n[r // G] > 0]
-            if ts:
-                kfin = max(k0[t] + n[t] for t in ts)
-                assert min(kfin - 1 + 127, C - 1) < C and min(k0[t] for t in ts) >= 0
-                assert all(n[t] <= maxk and t * H + hk * G + G - 1 < T * H for t in ts)
-        # wsum_kernel: R rows, one first key at a time
-        wide = (rows + 31) // 32 * Hkv >= 256
-        R, KC = (32, 64) if wide else (8, D)
-        for rho0 in range(0, rows, R):
-            tile = [(k0[r // G], n[r // G]) for r in range(rho0, min(rho0 + R, rows))]
-            assert all(0 <= head(hk, rho0 + i) < T * H for i in range(R))  # a row past the last: the last one's
-            for first in {k for k, c in tile if c > 0}:
-                nall = max(c for k, c in tile if k == first)
-                off, nblk = first % 8, (first % 8 + nall + 7) // 8
-                assert first // 8 + nblk - 1 < vblocks  # value blocks, clamped to the last
-                assert nall - 1 < maxk                  # scores, clamped to the row's last
-                assert (off + nall + KC - 1) // KC * KC >= off + nall
