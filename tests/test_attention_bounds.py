@@ -1,16 +1,17 @@
 """Host-side range check of the attention kernels' address arithmetic.
 
 Every global and LDS address that att_scores_kernel, att_decode_kernel,
-att_wsum_kernel, att_wsum_q4_kernel, att_scores_kpl_kernel and
-att_wsum_qpl_kernel (mimir-model_amd/csrc/decoder_ops.hip)
-compute is restated here per workgroup of the launch grid that
-launch_attention picks, and its extremes are checked against the sizes of
+att_wsum_kernel and att_wsum_q4_kernel (mimir-model_amd/csrc/decoder_ops.hip)
+and am::scores_kernel, am::wsum_kernel and am::decode_scores_kernel
+(attention_mfma.hip) compute is restated here per workgroup of the launch grid
+that launch_attention picks, and its extremes are checked against the sizes of
 the buffers: the key cache [kv_heads][C][D], the value cache blocked by eight
 keys [kv_heads][ceil(C/8)][D][8], q and out [T][H][D], the workspace
 [T][H][max_keys], and each kernel's LDS. The visible ranges come from
 adversarial end/start indices (negative, past C, past max_keys, empty
 ranges), over D = 8..512, one to many queries, slots, max_keys up to the
-8192 limit. CPU only: nothing here runs a kernel."""
+8192 limit. With the clamps of the restatement taken out the checks fail.
+CPU only: nothing here runs a kernel."""
 import itertools
 
 import numpy as np
@@ -25,6 +26,10 @@ def att_range(kend, kstart, t, C, maxk):
     n = int(kend[t]) + 1 - k0
     n = min(n, C - k0, maxk)
     return k0, max(n, 0)
+
+
+def clamp(v, hi):
+    return min(v, hi)
 
 
 class Bounds:
@@ -164,97 +169,139 @@ def check_wsum_q4(b, ranges):
                     assert 8 * nblk <= VS and offc + rows <= VS
 
 
-def check_scores_kpl(b, ranges):
-    """att_scores_kpl_kernel: workgroup (x, h, z) walks tiles of 256 cache
-    entries from the smallest first entry of its 32 queries, gridDim.x
-    apart; thread i reads key kb + i (clamped to the cache), stores the
-    score of key j = kb + i - k0 for 0 <= j < n."""
-    D, C, QG = b.D, b.C, 32
-    assert QG * D * 4 <= 64 * 1024  # the query rows in LDS
-    gx = (b.maxk + 255) // 256
-    for z in range((b.T + QG - 1) // QG):
-        r = [ranges[QG * z + i] if QG * z + i < b.T else (0, 0) for i in range(QG)]
-        live = [(k0, n) for k0, n in r if n > 0]
-        if not live:
-            continue
-        kmin = min(k0 for k0, _ in live)
-        kfin = max(k0 + n for k0, n in live)
-        for h in range(b.H):
-            hk = h // (b.H // b.Hkv)
-            for x in range(gx):
-                kb = kmin + 256 * x
-                while kb < kfin:
-                    a_lo, a_hi = min(kb, C - 1), min(kb + 255, C - 1)
-                    b.check((hk * C + a_lo) * D, (hk * C + a_hi) * D + D - 1, b.kc_len, "scores_kpl: key element")
-                    for i, (k0, n) in enumerate(r):
-                        if n <= 0:
-                            continue
-                        j_lo, j_hi = max(kb - k0, 0), min(kb + 255 - k0, n - 1)
-                        if j_lo > j_hi:
-                            continue
-                        t = QG * z + i
-                        assert t < b.T and j_hi < b.maxk
-                        b.check((t * b.H + h) * b.maxk + j_lo, (t * b.H + h) * b.maxk + j_hi, b.ws_len,
-                                "scores_kpl: out")
-                    kb += 256 * gx
+def row_of(b, ranges, hk, rho):
+    """am::row_of: first key, keys (none past the last row), t * H + h."""
+    G = b.H // b.Hkv
+    rows = b.T * G
+    rc = clamp(rho, rows - 1)
+    t = rc // G
+    k0, n = ranges[t] if rc == rho else (0, 0)
+    return k0, n, t * b.H + hk * G + rc - t * G
 
 
-def check_wsum_qpl(b, ranges):
-    """att_wsum_qpl_kernel: workgroup (h, z) of 16 queries; the scores of
-    each query (j < n) into LDS [key][16]; per pass (all queries when they
-    share the first entry, else one query at a time) the value blocks from
-    the block holding k0, four ahead and clamped to the last block, and the
-    LDS rows of keys below the pass's largest count."""
-    D, C, QG = b.D, b.C, 16
-    assert b.maxk * QG * 4 + 1024 <= LDS_BYTES
-    for z in range((b.T + QG - 1) // QG):
-        r = [ranges[QG * z + i] if QG * z + i < b.T else (0, 0) for i in range(QG)]
-        ns = [n for _, n in r]
-        for i, n in enumerate(ns):
-            assert n <= b.maxk
-            if n > 0:
-                assert QG * z + i < b.T
-        live = [i for i in range(QG) if ns[i] > 0]
-        if not live:
-            continue
-        same = all(r[i][0] == r[live[0]][0] for i in live)
-        passes = [live] if same else [[i] for i in live]
-        for h in range(b.H):
-            hk = h // (b.H // b.Hkv)
-            for qs in passes:
-                k0 = r[qs[0]][0]
-                nmax = max(ns[i] for i in qs)
+def check_scores_mfma(b, ranges):
+    """am::scores_kernel: 32 rows a workgroup, 32 keys a wave, tiles of 128
+    keys gridDim.y apart from the rows' first key on."""
+    D, C, G = b.D, b.C, b.H // b.Hkv
+    rows = b.T * G
+    xt = (rows + 31) // 32 * b.Hkv
+    gy = max(1, min(1024 // xt, ((C if b.kstart else b.maxk) + 127) // 128))
+    for hk in {0, b.Hkv - 1}:
+        for rho0 in range(0, rows, 32):
+            r = [row_of(b, ranges, hk, rho0 + i) for i in range(32)]
+            for i, (_, _, head) in enumerate(r):
+                if rho0 + i < rows:
+                    b.check(head * D, head * D + D - 1, b.T * b.H * D, "scores_mfma: q")
+                b.check(i * (D + 4), i * (D + 4) + D - 1, 32 * (D + 4), "scores_mfma: q row in LDS")
+            live = [x for x in r if x[1] > 0]
+            if not live:
+                continue
+            kmin, kfin = min(k0 for k0, _, _ in live), max(k0 + n for k0, n, _ in live)
+            walked = []
+            for y in range(gy):
+                for kt in range(kmin + 128 * y, kfin, 128 * gy):
+                    walked.append(kt)
+                    for w in range(4):
+                        kb = kt + 32 * w
+                        seen = [x for x in live if x[0] < kb + 32 and x[0] + x[1] > kb]
+                        if not seen:
+                            continue
+                        a_lo, a_hi = clamp(kb, C - 1), clamp(kb + 31, C - 1)
+                        b.check((hk * C + a_lo) * D, (hk * C + a_hi) * D + D - 1, (hk + 1) * C * D, "scores_mfma: key")
+                        for k0, n, head in seen:
+                            j_lo, j_hi = max(kb - k0, 0), min(kb + 31 - k0, n - 1)
+                            b.check(head * b.maxk + j_lo, head * b.maxk + j_hi, (head + 1) * b.maxk, "scores_mfma: out")
+            assert sorted(walked) == list(range(kmin, kfin, 128))  # every key's tile once
+            assert max(x[2] for x in live) < b.T * b.H
+
+
+def check_wsum_mfma(b, ranges, RT, each):
+    """am::wsum_kernel: RT rows and 64 dims a wave, one first key at a time."""
+    D, C, G = b.D, b.C, b.H // b.Hkv
+    rows, RG = b.T * G, 1 if each else 2
+    R, NT = RG * RT, RG * D
+    KC = 64 if RT == 16 else D
+    ES, HB = KC + 4, 4 if RT == 16 else KC // (16 if b.f16 else 32)
+    SEG = KC // 8 // HB
+    assert 8 * HB * SEG == KC and SEG % 2 == 0 and R * KC % NT == 0 and NT % KC in (0, NT) and KC % 64 == 0
+    assert 2 * R * ES * 4 + R * (8 + 8 + 1 + 1 + 1 + 1 + 1) * 4 <= LDS_BYTES // 2  # two workgroups a CU
+    b.check(0, (R - 1) * ES + 8 * HB * (SEG - 1) + 8 * HB - 1, R * ES, "wsum_mfma: weights read by the chains")
+    b.check(0, (R - 1) * ES + 7 + 8 * (KC // 8 - 1), R * ES, "wsum_mfma: weights read by the lane sums")
+    for hk in {0, b.Hkv - 1}:
+        for rho0 in range(0, rows, R):
+            r = [row_of(b, ranges, hk, rho0 + i) for i in range(R)]
+            for _, _, head in r:  # every row's scores are loaded, of a row without a key the first word
+                b.check(head * b.maxk, head * b.maxk, b.ws_len, "wsum_mfma: a row's first score")
+            for i, (_, n, head) in enumerate(r):
+                if rho0 + i < rows:
+                    b.check(head * D, head * D + D - 1, b.T * b.H * D, "wsum_mfma: out")
+                assert n == 0 or rho0 + i < rows
+            firsts = list(dict.fromkeys(k0 for k0, n, _ in r if n > 0))
+            if each:
+                assert len(firsts) <= (G + 2) // G + 1  # a workgroup for each
+            for k0 in firsts:
+                nall = max(n for k, n, _ in r if n > 0 and k == k0)
                 off = k0 & 7
-                kbeg = k0 - off
-                nblk = (off + nmax + 7) >> 3
-                last_blk = kbeg + 8 * (nblk - 1)
-                assert kbeg >= 0 and last_blk < ((C + 7) // 8) * 8
+                kbeg, nch, nblk = k0 - off, (off + nall + KC - 1) // KC, (off + nall + 7) >> 3
+                for k, n, head in r:
+                    un = n if k == k0 else 0
+                    # slots -off .. of the first chunk to the last one's end, and the last n % 8 keys
+                    for j in (-off, KC * (nch - 1) + KC - 1 - off, (un & ~7) + 7, nall + 63):
+                        at = max(clamp(j, un - 1), 0)
+                        b.check(head * b.maxk, head * b.maxk + at, (head + 1) * b.maxk, "wsum_mfma: scores")
+                last = clamp(HB * (SEG * (nch - 1) + SEG) + HB - 1, nblk - 1)  # one segment read ahead
                 for d in (0, D - 1):
-                    b.check(b.vcache_at(hk, kbeg, d), b.vcache_at(hk, last_blk, d) + 7, b.vc_len,
-                            "wsum_qpl: value element")
-                assert nmax - 1 < b.maxk  # LDS rows of the keys read
+                    b.check(b.vcache_at(hk, kbeg, d), b.vcache_at(hk, kbeg + 8 * last, d) + 7, b.vcache_at(hk + 1, 0, 0),
+                            "wsum_mfma: value block")
+                assert 8 * HB * SEG * nch >= off + nall  # every key's weight is in a chunk
 
 
-def run_launch(T, H, Hkv, D, C, maxk, f16, kend, kstart):
+def check_decode_scores(b, ranges):
+    """am::decode_scores_kernel: a wave per 64 keys, kv head and query."""
+    D, C, G = b.D, b.C, b.H // b.Hkv
+    PC, NG = D * b.esz // 16, 1 if G <= 4 else 2
+    sw = lambda k: k & (PC - 1) & 15
+    for k in range(64):  # the swizzle moves a key's pieces within the key
+        assert sorted(p ^ sw(k) for p in range(PC)) == list(range(PC))
+    b.check(0, 1024 * (PC - 1) + 16 * 63 + 15, 64 * PC * 16, "decode_scores: pieces in LDS")
+    b.check(0, (4 * NG - 1) * (D + 4) + D - 1, 4 * NG * (D + 4), "decode_scores: q rows in LDS")
+    for t, (k0, n) in enumerate(ranges):
+        for hk in {0, b.Hkv - 1}:
+            head0 = t * b.H + hk * G
+            for j0 in range(0, min(n, b.maxk), 64):
+                lo, hi = clamp(j0, n - 1), clamp(j0 + 63, n - 1)
+                b.check((hk * C + k0 + lo) * D, (hk * C + k0 + hi) * D + D - 1, (hk + 1) * C * D, "decode_scores: key")
+                heads = [head0 + 4 * g + i for g in range(NG) for i in range(4) if 4 * g + i < G]
+                b.check(min(heads) * D, (head0 + clamp(4 * NG - 1, G - 1)) * D + D - 1, b.T * b.H * D, "decode_scores: q")
+                j = min(j0 + 63, n - 1)
+                b.check(min(heads) * b.maxk + j0, max(heads) * b.maxk + j, (head0 + G) * b.maxk, "decode_scores: out")
+            assert n <= b.maxk
+
+
+def run_launch(T, H, Hkv, D, C, maxk, f16, kend, kstart, aligned=True):
     b = Bounds(T, H, Hkv, D, C, maxk, f16)
+    b.kstart = kstart is not None
     ranges = [att_range(kend, kstart, t, C, maxk) for t in range(T)]
     for k0, n in ranges:
         assert 0 <= k0 < C and 0 <= n <= min(C - k0, maxk)
-    many = T >= 16 and D % 64 == 0 and maxk <= 2048
-    if many and T >= 256 and (D == 64 or (D == 128 and f16)) and maxk <= 1024:
-        check_scores_kpl(b, ranges)
-        check_wsum_qpl(b, ranges)
-        return "prompt"
-    if many:
+    G = H // Hkv
+    if T >= 16 and D in (64, 128) and aligned:
+        check_scores_mfma(b, ranges)
+        each = b.kstart and G <= 4 and T * G * maxk <= 4 * C
+        RT = 16 if (T * G + 31) // 32 * Hkv >= 256 and not each else 4
+        check_wsum_mfma(b, ranges, RT, each)
+        return "each" if each else f"mfma{RT}"
+    if T >= 16 and D % 64 == 0 and maxk <= 2048:
         check_scores(b, ranges, 4)
         check_wsum_q4(b, ranges)
         return "many"
     if D in (64, 128) and maxk <= ATT_DEC_MAXK:
         check_decode(b, ranges)
         return "decode"
-    # (att_scores_gqa_kernel, taken for D 64/128 and 2/4/8 query heads per
-    # kv head, reads the same key rows per tile and writes the same score
-    # rows as the per-head kernel checked here)
+    if D in (64, 128) and 2 <= G <= 8 and aligned and (maxk + 63) // 64 * Hkv * T >= 256:
+        check_decode_scores(b, ranges)
+        check_wsum(b, ranges)
+        return "two_grouped"
     check_scores(b, ranges, 1)
     check_wsum(b, ranges)
     return "two"
@@ -282,19 +329,38 @@ def ranges_for(T, C, maxk, slots, rng):
 def test_attention_addresses_in_bounds(D, f16):
     rng = np.random.default_rng(D + (1000 if f16 else 0))
     seen = set()
-    for T, (H, Hkv), C, slots, maxk_kind in itertools.product(
-            (1, 3, 8, 16, 37, 300), ((4, 1), (8, 2), (4, 4)), (1, 7, 42, 301, 2048, 8200), (1, 3),
-            ("C", "small", "max")):
-        if slots > C:
+    for T, (H, Hkv), C, slots, maxk_kind, aligned in itertools.product(
+            (1, 3, 8, 16, 37, 300), ((4, 1), (8, 2), (4, 4), (32, 8)), (1, 7, 42, 301, 2048, 8200), (1, 3, 40),
+            ("C", "slot", "small", "max"), (True, False)):
+        if slots > C or (H == 32 and T != 300) or (not aligned and (D not in (64, 128) or C > 301)):
             continue
-        maxk = {"C": min(C, 8192), "small": max(1, min(C, 8192) // 3), "max": 8192}[maxk_kind]
-        if T * maxk > 8 * 8192 * 37:
+        if (slots == 40) != (maxk_kind == "slot") or (slots == 40 and D not in (64, 128)):
+            continue
+        maxk = {"C": min(C, 8192), "slot": min(C // slots, 8192), "small": max(1, min(C, 8192) // 3), "max": 8192}[maxk_kind]
+        if T * maxk > 8 * 8192 * 37 or (H == 32 and maxk > 2048):
             continue
         kend, kstart = ranges_for(T, C, maxk, slots, rng)
-        seen.add(run_launch(T, H, Hkv, D, C, maxk, f16, kend, kstart if slots > 1 or T > 5 else None))
-    if D == 64 or (D == 128 and f16):
-        assert seen == {"many", "decode", "two", "prompt"}
-    elif D == 128:
-        assert seen == {"many", "decode", "two"}
+        seen.add(run_launch(T, H, Hkv, D, C, maxk, f16, kend, kstart if slots > 1 or T > 5 else None, aligned))
+    if D in (64, 128):
+        assert seen == {"mfma4", "mfma16", "each", "many", "decode", "two", "two_grouped"}
     elif D % 64 == 0:
         assert seen == {"many", "two"}
+    else:
+        assert seen == {"two"}
+
+
+@pytest.mark.parametrize("T,H,Hkv,C,slots,maxk,path", [(37, 4, 4, 301, 1, 301, "mfma4"), (300, 32, 8, 301, 1, 301, "mfma16"),
+                                                      (37, 4, 4, 37 * 20, 37, 20, "each"), (8, 8, 2, 2047, 1, 2047, "two_grouped")])
+def test_missing_clamps_are_found(monkeypatch, T, H, Hkv, C, slots, maxk, path):
+    """The checks of the matrix-core kernels fail when the restatement's
+    clamps (rows past the last, keys and value blocks past the end) go."""
+    rng = np.random.default_rng(T)
+    for t0 in range(3):
+        kend, kstart = ranges_for(T, C, maxk, slots, rng)
+        kend[-1], kstart[-1] = C - 1, max(0, C - maxk)
+        args = (T, H, Hkv, 64, C, maxk, True, kend, kstart if slots > 1 else None)
+        assert run_launch(*args) == path
+        with monkeypatch.context() as m:
+            m.setitem(globals(), "clamp", lambda v, hi: v)
+            with pytest.raises((AssertionError, IndexError)):
+                run_launch(*args)
