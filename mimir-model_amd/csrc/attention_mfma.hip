@@ -523,9 +523,6 @@ __global__ __launch_bounds__((EACH ? 1 : 2) * D, 2) void wsum_kernel(Args A) {
 // Measured on MI355X, us, the whole attention, against a workgroup per 64 keys
 // with eight lanes a key on the vector unit: that size 33.9 -> 32.4; 64 heads
 // of 8 kv heads, 300 keys 23.2 -> 20.5; 24 of 4, D = 64, 2000 keys 22.8 -> 19.6.
-__device__ __forceinline__ void lds_copy16(const void* g, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(g), "s"(lds) : "memory");
-}
 
 template <bool F16, int D, int NG>
 __global__ __launch_bounds__(64) void decode_scores_kernel(Args A) {

@@ -89,14 +89,6 @@ struct Smem {
     int wbad[NCW];
 };
 
-// Global -> LDS copy of 16 bytes a lane (lane i writes at lds + 16 i). Inline
-// assembly, so that the compiler does not wait for the copies in flight; the
-// copy waves wait for them explicitly (WAIT_VMCNT).
-__device__ __forceinline__ void copy16(const void* g, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(g),
-                 "s"(__builtin_amdgcn_readfirstlane(lds))
-                 : "memory", "m0");
-}
 #define CH_WAIT_VMCNT(n) __builtin_amdgcn_s_waitcnt(((n) & 0xF) | (((n) >> 4) << 14) | (0x7 << 4) | (0xF << 8))
 
 // A workgroup barrier that waits for nothing in flight (the copy waves'
@@ -225,7 +217,7 @@ __device__ __forceinline__ void issue_stage(const ChainArgs& A, const StageD& s,
         const int qi = cw + NCP * k;
         int64_t off = (int64_t)qi * 1024 + 16 * lane;
         if (off > bytes - 16) off = bytes - 16;
-        copy16(base + off, ring0 + (uint32_t)(slot * SB + qi * 1024));
+        lds_copy16(base + off, __builtin_amdgcn_readfirstlane(ring0 + (uint32_t)(slot * SB + qi * 1024)));
     }
 }
 

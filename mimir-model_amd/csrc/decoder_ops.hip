@@ -144,7 +144,6 @@ __global__ void rope_kernel(float* __restrict__ x, const int64_t* __restrict__ p
     }
 }
 
-
 // k, v [T][Hkv][D] into the caches at the cache indices pos[t] (rounded to
 // f16 when the cache is f16).
 __global__ void kv_store_kernel(const float* __restrict__ k, const float* __restrict__ v, const int64_t* __restrict__ pos,
@@ -167,7 +166,6 @@ __global__ void kv_store_kernel(const float* __restrict__ k, const float* __rest
         }
     }
 }
-
 
 // rope.v1 on q and k and the cache scatter of k and v in one launch (the
 // graph's rope of q and k and its cache update, importer/llama.go:364-503):
@@ -838,13 +836,6 @@ __global__ __launch_bounds__(256) void att_wsum_q4_kernel(const void* vc, const 
 // The float steps and their order are those of the reference's attendRow
 // (attn_amd64.s): the chain per dim in key order, the eight-lane exp sum.
 
-// Global -> LDS copy of 16 bytes a lane (lane i writes at the wave's LDS
-// base + 16i), written as inline assembly so that the compiler does not
-// count it: the copying waves' waits are explicit (ATT_WAIT_VMCNT).
-__device__ __forceinline__ void att_lds_copy16(const void* g, const void* lds_wave_base) {
-    const uint32_t m0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)lds_wave_base);
-    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(g), "s"(m0) : "memory", "m0");
-}
 // s_waitcnt with vmcnt <= n (n < 64), the other counters unconstrained.
 #define ATT_WAIT_VMCNT(n) __builtin_amdgcn_s_waitcnt(((n) & 0xF) | (((n) >> 4) << 14) | (0x7 << 4) | (0xF << 8))
 
@@ -854,7 +845,6 @@ __device__ __forceinline__ void att_barrier() {  // s_barrier without __syncthre
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
 }
-
 
 template <bool F16>
 constexpr int att_bb() {  // blocks of 8 keys per batch
@@ -909,7 +899,7 @@ __global__ __launch_bounds__(256) void att_wsum_kernel(const void* vc, const int
         for (int ii = 0; ii < CPB; ii++) {
             const int i = F16 ? 2 * ii + cw : ii;
             const int b = BB * k + i < nb ? BB * k + i : nb - 1;
-            att_lds_copy16(vsrc + b * bstride, slot + i * PPB * 1024);
+            lds_copy16(vsrc + b * bstride, slot + i * PPB * 1024);
         }
     };
     if (copier)
@@ -1218,7 +1208,6 @@ static void launch_att_scores(dim3 grid, const float* q, const void* kc, const i
         hipLaunchKernelGGL((att_scores_kernel<F16, 0, QT>), grid, dim3(256), 0, s, q, kc, kend, kstart, T, H, Hkv, D, C,
                            maxk, ws);
 }
-
 
 hipError_t launch_attention(const float* q, const void* kc, const void* vc, const int64_t* kend, const int64_t* kstart,
                             int T, int H, int Hkv, int D, int64_t C, int64_t maxk, int f16, float* out, float* ws,

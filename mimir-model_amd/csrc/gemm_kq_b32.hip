@@ -89,20 +89,6 @@ struct Args {
     int tiles_m;
 };
 
-__device__ __forceinline__ uint32_t lds_addr(const void* p) {
-    return __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)p);
-}
-// global_load_lds copies (lane i writes its bytes at the wave's LDS base +
-// 16i or 4i), written as inline assembly so that the compiler does not wait
-// for them at every LDS read; the waits are explicit.
-__device__ __forceinline__ void lds_copy16(const void* g, uint8_t* lds_wave_base) {
-    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(g), "s"(lds_addr(lds_wave_base))
-                 : "memory", "m0");
-}
-__device__ __forceinline__ void lds_copy4(const void* g, uint8_t* lds_wave_base) {
-    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(g), "s"(lds_addr(lds_wave_base))
-                 : "memory", "m0");
-}
 #define KQ_WAIT_VMCNT(n) __builtin_amdgcn_s_waitcnt(((n) & 0xF) | (((n) >> 4) << 14) | (0x7 << 4) | (0xF << 8))
 #define KQ_WAIT_LGKM0() __builtin_amdgcn_s_waitcnt(0xC07F)
 __device__ __forceinline__ void kq_barrier() {

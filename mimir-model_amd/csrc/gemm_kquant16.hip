@@ -89,25 +89,6 @@ struct GemmArgs {
     int fused;             // float32 fallback order (rows of the whole call <= 8)
 };
 
-// Global -> LDS copies (global_load_lds: lane i of the wave writes its 16
-// or 4 bytes at the wave's LDS base + 16i or 4i). Written as inline
-// assembly so that the compiler does not track them: it would otherwise wait
-// for every copy in flight (vmcnt(0)) before the first LDS read of a block,
-// including the next block's prefetch. The waits are explicit instead
-// (GM_WAIT_VMCNT), and the compiler's own waits can only be stronger, the
-// counter retiring in order.
-__device__ __forceinline__ uint32_t lds_addr(const void* p) {
-    return __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)p);
-}
-__device__ __forceinline__ void lds_copy16(const void* g, uint8_t* lds_wave_base) {
-    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(g), "s"(lds_addr(lds_wave_base))
-                 : "memory", "m0");
-}
-__device__ __forceinline__ void lds_copy4(const void* g, uint8_t* lds_wave_base) {
-    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(g), "s"(lds_addr(lds_wave_base))
-                 : "memory", "m0");
-}
-
 // s_waitcnt with vmcnt <= n (n < 64) and the other counters unconstrained.
 #define GM_WAIT_VMCNT(n) __builtin_amdgcn_s_waitcnt(((n) & 0xF) | (((n) >> 4) << 14) | (0x7 << 4) | (0xF << 8))
 // s_waitcnt lgkmcnt(0) (LDS reads of this wave done).

@@ -93,16 +93,6 @@ struct Args {
     int tiles_m;           // row tiles of BM activation rows
 };
 
-// global_load_lds: lane i of the wave writes its 16 (4) bytes at the wave's
-// LDS base + 16i (4i). Inline assembly, so that the compiler does not wait
-// for the copies in flight at every LDS read; the waits are explicit, and
-// the compiler's own can only be stronger (the counter retires in order).
-__device__ __forceinline__ void lds_copy16(const void* g, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(g), "s"(lds) : "memory");
-}
-__device__ __forceinline__ void lds_copy4(const void* g, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(g), "s"(lds) : "memory");
-}
 // s_waitcnt with vmcnt <= n (n < 64), the other counters unconstrained.
 #define GQ4_WAIT_VMCNT(n) __builtin_amdgcn_s_waitcnt(((n) & 0xF) | (((n) >> 4) << 14) | (0x7 << 4) | (0xF << 8))
 

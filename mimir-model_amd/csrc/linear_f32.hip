@@ -116,21 +116,6 @@ __device__ __forceinline__ void vdecode(const VRaw& r, int v, float (&out)[8]) {
     }
 }
 
-__device__ __forceinline__ uint32_t lds_addr(const void* p) {
-    return __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)p);
-}
-// global_load_lds copies: lane i's 16 (or 4) bytes land at the wave's LDS
-// base + 16 i (4 i). Inline assembly, so that the compiler does not wait for
-// them at every LDS read; the wait is the vmcnt(0) before the barrier.
-__device__ __forceinline__ void lds_copy16(const void* g, float* lds_wave_base) {
-    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(g), "s"(lds_addr(lds_wave_base))
-                 : "memory");
-}
-__device__ __forceinline__ void lds_copy4(const void* g, float* lds_wave_base) {
-    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(g), "s"(lds_addr(lds_wave_base))
-                 : "memory");
-}
-
 template <int WM>
 struct Tile {
     static constexpr int T = 256 * WM, BM = 32 * WM;

@@ -54,13 +54,6 @@ __device__ __forceinline__ u32x4 load16_a2(const uint8_t* p) {
     return r;
 }
 
-// 4 bytes starting at a 2-byte-aligned address.
-__device__ __forceinline__ uint32_t load4_a2(const uint8_t* p) {
-    const uint32_t* b = (const uint32_t*)__builtin_align_down(p, 4);
-    uint32_t s = (uint32_t)((uintptr_t)p & 3);
-    return __builtin_amdgcn_alignbyte(b[1], b[0], s);
-}
-
 __device__ __forceinline__ uint16_t load_u16(const uint8_t* p) { return *(const uint16_t*)p; }
 
 __device__ __forceinline__ int sdot4(uint32_t a, uint32_t b, int c) {
@@ -135,6 +128,23 @@ __device__ __forceinline__ void lds_barrier() {
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
+
+// Global -> LDS copies: lane i of the wave writes its 16 (4) bytes at the
+// wave's LDS base + 16i (4i); the base comes through m0. Inline assembly, so
+// that the compiler does not wait for the copies in flight at every LDS read:
+// the kernel waits for them itself (s_waitcnt vmcnt), and the compiler's own
+// waits can only be stronger, the counter retiring in order.
+__device__ __forceinline__ uint32_t lds_addr(const void* p) {
+    return __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)p);
+}
+__device__ __forceinline__ void lds_copy16(const void* g, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(g), "s"(lds) : "memory", "m0");
+}
+__device__ __forceinline__ void lds_copy4(const void* g, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(g), "s"(lds) : "memory", "m0");
+}
+__device__ __forceinline__ void lds_copy16(const void* g, const void* lds) { lds_copy16(g, lds_addr(lds)); }
+__device__ __forceinline__ void lds_copy4(const void* g, const void* lds) { lds_copy4(g, lds_addr(lds)); }
 
 // Whether p holds on any thread of the workgroup's nw waves: one LDS flag
 // per wave (slot[nw], written once per launch) and one LDS-only barrier.
