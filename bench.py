@@ -67,7 +67,6 @@ compared with the GPU's (8 tokens; the 8B shape on a 32-token prompt).
 import argparse
 import ctypes
 import json
-import math
 import os
 import platform
 import sys
@@ -106,6 +105,12 @@ def weight_bytes(n, k, dt):
 
 def step_bytes(rows=1):
     return sum(weight_bytes(n, k, dt) + rows * (k * 4 + n * 4) for _, n, k, dt, _, _ in CFG1)
+
+
+def step_pieces(steps, most, rotate):
+    """`steps` steps from rotation layer 0 on as runs of at most `most`
+    consecutive ones: [(first layer, count)]."""
+    return [(s % rotate, min(most, steps - s)) for s in range(0, steps, most)]
 
 
 def launch_bytes(n, k, dt, rows=1):
@@ -351,8 +356,7 @@ def main():
                          "one launch per grouped call, as a decoder layer makes them; chain: the four grouped "
                          "products as one chain launch (mimg_linear_a8_chain_dev, one row only)")
     ap.add_argument("--graph-steps", type=int, default=0,
-                    help="steps captured in one HIP graph (consecutive rotation layers; divides --rotate; "
-                         "default: the largest that divides --rotate, --steps and --warmup)")
+                    help="most steps captured in one HIP graph (consecutive rotation layers; default: --rotate)")
     ap.add_argument("--roofline-replays", type=int, default=8,
                     help="replays of the graph of --rotate single-kernel launches timed for the roofline")
     args = ap.parse_args()
@@ -500,55 +504,56 @@ def main():
                 mimg.linear_a8_group_dev([layers[l][c[0]] for c in grp], xd[i].ptr, M, None, 256,
                                          [yd[c[0]].ptr for c in grp], ws[i].ptr, ws_bytes[i], stream.handle)
 
-    # A graph holds gs consecutive steps (layers l .. l+gs-1 of the rotation:
-    # all 32 at the default --steps and --warmup, one token's linear sets, as a
-    # decode step's graph holds all of a token's layers); with gs = 1 the host
-    # launches one graph per step.
-    gs = args.graph_steps or math.gcd(args.rotate, args.steps, args.warmup)
-    if args.rotate % gs or args.steps % gs or args.warmup % gs:
-        raise SystemExit("--graph-steps must divide --rotate, --steps and --warmup")
-    if args.eager:
-        gs = 1
+    # A graph holds up to gs consecutive steps (all 32 rotation layers, one
+    # token's linear sets, as a decode step's graph holds all of a token's
+    # layers) whatever --steps and --warmup are: the last one of either holds
+    # what is left.
+    gs = 1 if args.eager else args.graph_steps or args.rotate
+    if gs < 1:
+        raise SystemExit("--graph-steps must be at least 1")
 
     def time_steps(kind):
         """Warm-up, then exactly --steps steps of `kind` between two events
         on the launch stream (and device synchronisations); us per step and
         the wall time per step."""
-        graphs = []
-        if args.eager:
-            def run(l):
-                enqueue_step(kind, l)
-        else:
-            def enqueue_steps(l0):
-                for l in range(l0, l0 + gs):
-                    enqueue_step(kind, l)
+        graphs = {}
 
-            graphs = [hiprt.Graph(stream, lambda l0=l0: enqueue_steps(l0)) for l0 in range(0, args.rotate, gs)]
+        def enqueue_steps(first, count):
+            for l in range(first, first + count):
+                enqueue_step(kind, l % args.rotate)
 
-            def run(l):
-                graphs[l // gs].launch(stream)
+        def run(piece):
+            if args.eager:
+                enqueue_steps(*piece)
+            else:
+                graphs[piece].launch(stream)
 
-        for s in range(0, args.warmup, gs):
-            run(s % args.rotate)
+        warm, timed = step_pieces(args.warmup, gs, args.rotate), step_pieces(args.steps, gs, args.rotate)
+        if not args.eager:
+            for piece in dict.fromkeys(warm + timed):
+                graphs[piece] = hiprt.Graph(stream, lambda piece=piece: enqueue_steps(*piece))
+                graphs[piece].upload(stream)  # not on the first, timed launch
+        for piece in warm:
+            run(piece)
         stream.sync()
         e0, e1 = hiprt.Event(), hiprt.Event()
         hiprt.device_sync()
         t0 = time.perf_counter()
         e0.record(stream)
-        for s in range(0, args.steps, gs):
-            run(s % args.rotate)
+        for piece in timed:
+            run(piece)
         e1.record(stream)
         e1.sync()
         hiprt.device_sync()
         wall = time.perf_counter() - t0
         us = e0.elapsed_ms(e1) * 1e3 / args.steps
-        for g in graphs:
+        for g in graphs.values():
             g.destroy()
         if kind == "chain":
             st = mimg.chain_status(sync.ptr)
             if st:
                 raise SystemExit(f"chain status {st}: a device barrier wait timed out")
-        log(f"  timed ({kind}, {gs} steps a graph): {args.steps} steps, {us:.2f} us/step (events), "
+        log(f"  timed ({kind}, up to {gs} steps a graph): {args.steps} steps, {us:.2f} us/step (events), "
             f"wall {wall * 1e6 / args.steps:.2f} us/step, {step_bytes(M) / (us * 1e-6) / 1e9:.1f} GB/s")
         return us
 
@@ -836,7 +841,7 @@ def main():
             "bytes_per_step": step_bytes(M),
             "rotation_layers": args.rotate,
             "graphs": not args.eager,
-            "steps_per_graph": gs,
+            "steps_per_graph": min(gs, args.steps),
             "other_forms_us_per_step": other_us,
             "hbm_fraction": round(value / HBM_PEAK_GBS, 4),
         },

@@ -174,6 +174,10 @@ class Graph:
         check(rt().hipGraphInstantiate(ctypes.byref(ge), ctypes.c_void_p(self.graph), None, None, 0), "hipGraphInstantiate")
         self.exec = ge.value
 
+    def upload(self, stream):
+        """Brings the executable graph to the device ahead of its first launch."""
+        check(rt().hipGraphUpload(ctypes.c_void_p(self.exec), ctypes.c_void_p(stream.handle)), "hipGraphUpload")
+
     def launch(self, stream):
         check(rt().hipGraphLaunch(ctypes.c_void_p(self.exec), ctypes.c_void_p(stream.handle)), "hipGraphLaunch")
 
