@@ -2,7 +2,7 @@
 the C restatement, bit for bit: the GEMV up to 8 rows and the matrix-core
 tiles above, at ragged rows and weight rows around their tiles (8 weight rows;
 32 x 32 and 32 x 64), one and several stages of K, Q8_0 rows that end inside a
-stage, and non-finite activations and scales."""
+stage, non-finite activations and scales, and the value classes of a chain."""
 import numpy as np
 import pytest
 
@@ -45,10 +45,64 @@ def test_rows_and_tiles(gpu, oracle, dt, k, rows, n):
 def test_non_finite(gpu, oracle, dt, rows):
     def edit(wb, x):
         x[0, 5], x[1, 7], x[2, 3] = np.inf, np.nan, -np.inf
-        x[2, 100:140] = 1e-42  # subnormal products
         w = wb.reshape(40, -1)
         at = {Q4_K: 0, Q6_K: 208, Q8_0: 0}[dt]
         w[4, at:at + 2] = np.frombuffer(np.float16(np.inf).tobytes(), np.uint8)
         w[9, at:at + 2] = np.frombuffer(np.float16(np.nan).tobytes(), np.uint8)
 
     check(gpu, oracle, dt, 40, 768, rows, seed=3, edit=edit)
+
+
+@pytest.mark.parametrize("dt", [Q4_K, Q6_K, Q8_0])
+@pytest.mark.parametrize("rows", [3, 40])
+def test_subnormal(gpu, oracle, dt, rows):
+    """Rows whose products, sums and outputs are all subnormal: subnormal
+    activations, and small normal ones."""
+    n, k = 40, 768
+    wb = oracle.synthetic_weight(dt, n, k, seed=5)
+    x = oracle.synthetic_acts(rows, k, seed=6) * np.float32(1e-39)
+    x[1::2] *= np.float32(0.01)
+    W = gpu.Weight(wb, dt, n, k)
+    got = gpu.dequant_matmul(W, x)
+    W.release()
+    want = oracle.linear_f32(x, wb, dt, n, k, threads=8)
+    assert np.all(np.abs(want) < np.finfo(np.float32).tiny) and np.count_nonzero(want) > want.size // 2
+    assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+
+
+def _bits(rng, exponents, shape):
+    """Floats of random sign and mantissa, biased exponents from a range."""
+    e = rng.integers(*exponents, shape, dtype=np.uint32)
+    return (rng.integers(0, 1 << 23, shape, dtype=np.uint32) | e << 23 | rng.integers(0, 2, shape, dtype=np.uint32) << 31).view(np.float32)
+
+
+@pytest.mark.parametrize("exponents", [(0, 255), (0, 30), (90, 160), (225, 255)], ids=["all", "tiny", "middle", "huge"])
+def test_matrix_core_chain_is_fma(gpu, oracle, exponents):
+    """A chain on v_mfma_f32_32x32x1 against the same chain on the vector
+    unit's fmaf: for Q8_0 weights the rows of one call of 40 (matrix cores)
+    have the steps of calls of at most 8 (fmaf). Every value class of the
+    activations, f16 scales of every finite class; a row with one NaN keeps
+    its sign and payload (several NaNs: which one survives is the adds')."""
+    n, k, rows = 70, 1056, 40
+    rng = np.random.default_rng(exponents[0] * 1000 + exponents[1])
+    wb = rng.integers(0, 256, (n, k // 32, 34), dtype=np.uint8)
+    d = rng.integers(0, 0x7C00, (n, k // 32), dtype=np.uint16) | rng.integers(0, 2, (n, k // 32), dtype=np.uint16) << 15
+    wb[:, :, :2] = d.astype("<u2").view(np.uint8).reshape(n, k // 32, 2)
+    x = _bits(rng, exponents, (rows, k))
+    x[3, 7], x[4, 100] = np.inf, -np.inf
+    nans = {5: (1000, 0x7FC12345), 6: (31, 0xFFC00001), 7: (0, 0x7FABCDEF), 39: (1055, 0x7FFFFFFF)}
+    for m, (c, u) in nans.items():
+        x[m] = _bits(rng, (90, 130), k)  # no other NaN arises in the row
+        x.view(np.uint32)[m, c] = u
+    W = gpu.Weight(wb.reshape(-1), Q8_0, n, k)
+    got = gpu.dequant_matmul(W, x)
+    want = np.concatenate([gpu.dequant_matmul(W, np.ascontiguousarray(x[m:m + 8])) for m in range(0, rows, 8)])
+    W.release()
+    ok = np.isnan(got) & np.isnan(want)
+    ok[list(nans)] = False
+    same = (got.view(np.uint32) == want.view(np.uint32)) | ok
+    assert same.all(), f"{(~same).sum()} of {same.size} differ, first at {np.argwhere(~same)[0]}"
+    assert np.isnan(got[list(nans)]).all()
+    ref = oracle.linear_f32(x, wb.reshape(-1), Q8_0, n, k, threads=8)
+    same = (got.view(np.uint32) == ref.view(np.uint32)) | (np.isnan(got) & np.isnan(ref))
+    assert same.all(), f"{(~same).sum()} of {same.size} differ from the oracle"

@@ -43,3 +43,18 @@ def test_refusals(gpu, oracle, rows, n):
         x[rows - 1, 100] = np.float32(1e30)
 
     check(gpu, oracle, rows, n, 512, edit=edit, bias=True)
+
+
+@pytest.mark.parametrize("rows,n", [(100, 3100), (300, 7000)])
+def test_subnormal_scale_products(gpu, oracle, rows, n):
+    """Scale products d * dx and dmin * dx that are subnormal, zero or among
+    the smallest normal numbers: the outer product on the matrix cores rounds
+    them as the multiplication does."""
+    def edit(wb, x):
+        rng = np.random.default_rng(n)
+        blocks = wb.reshape(n, 2, 144)
+        d = rng.integers(0, 0x0800, (n, 2, 2), dtype=np.uint16)  # f16 up to 2^-13, subnormal ones among them
+        blocks[:, :, :4] = d.astype("<u2").view(np.uint8).reshape(n, 2, 4)
+        x *= (10.0 ** rng.uniform(-38, -28, (rows, 1))).astype(np.float32)
+
+    check(gpu, oracle, rows, n, 512, edit=edit)
