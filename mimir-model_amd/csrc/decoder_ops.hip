@@ -1214,15 +1214,27 @@ hipError_t launch_attention(const float* q, const void* kc, const void* vc, cons
                             hipStream_t s) {
     if (D > 512 || D % 8 || H % Hkv || maxk < 1 || maxk > ATT_MAXC || T < 1) return hipErrorInvalidValue;
     const unsigned tiles = (unsigned)((maxk + 63) / 64);
-    // from 16 queries at D = 64 or 128: the matrix cores (measured on MI355X
-    // at 32 heads, D = 128: 16 queries of 64 keys 16.7 -> 13.9 us, of 2048
-    // keys 32 -> 14). C below 2^30: its 32-bit key indices.
-    if (T >= 16 && (D == 64 || D == 128) && C < (1 << 30) &&
-        (((uintptr_t)q | (uintptr_t)kc | (uintptr_t)vc) & 15) == 0)
+    // D = 64 or 128, at most ATT_DEC_MAXK keys, few queries: one launch of
+    // T * H * D / 32 workgroups (att_decode_kernel). Its workgroups compute all of a query's
+    // scores each, which beats the two-kernel paths only for short contexts
+    // (measured on MI355X at D = 128, one query: 4.7 against 7.5 us at 64 keys,
+    // 17.9 against 13.6 at 640) and, from 16 queries on, only for small grids:
+    // against the matrix cores' two launches 0.36 to 1.00 of the time up to 512
+    // workgroups at 64, 128 and 256 keys (2 heads, 26 queries, D = 128: 5.9 for
+    // 15.0 us), 0.40 to 0.72 up to 1024 at 64 keys; 0.43 to 1.34 from 512 to
+    // 1024 at 256 keys, 0.61 to 1.16 from 1536 to 2048 at 64.
+    const bool al16 = (((uintptr_t)q | (uintptr_t)kc | (uintptr_t)vc) & 15) == 0;
+    const int64_t decw = (int64_t)T * H * (D / 32);
+    const bool dec = (D == 64 || D == 128) && maxk <= ATT_DEC_MAXK && T <= 65535 &&
+                     (T < 16 || (al16 && (decw <= 512 || (decw <= 1024 && maxk <= 64))));
+    // otherwise from 16 queries on: the matrix cores (measured on MI355X at 32
+    // heads, D = 128: 16 queries of 64 keys 16.7 -> 13.9 us, of 2048 keys 32 ->
+    // 14). C below 2^30: its 32-bit key indices.
+    if (T >= 16 && !dec && (D == 64 || D == 128) && C < (1 << 30) && al16)
         return launch_attention_mfma(q, kc, vc, kend, kstart, T, H, Hkv, D, C, maxk, f16, out, ws, s);
     // many queries of other sizes: four per workgroup, sharing the key and
     // value loads
-    const bool many = T >= 16 && D % 64 == 0 && maxk <= 2048;
+    const bool many = T >= 16 && !dec && D % 64 == 0 && maxk <= 2048;
     if (many) {
         const dim3 grid(tiles, (unsigned)H, (unsigned)((T + 3) / 4));
         if (f16) launch_att_scores<true, 4>(grid, q, kc, kend, kstart, T, H, Hkv, D, C, maxk, ws, s);
@@ -1237,12 +1249,7 @@ hipError_t launch_attention(const float* q, const void* kc, const void* vc, cons
                                ws, out);
         return hipGetLastError();
     }
-    // few queries, D = 64 or 128, at most ATT_DEC_MAXK keys: one launch per
-    // query (att_decode_kernel). Its workgroups compute all of a query's
-    // scores each, which beats the two-kernel path (scores spread over
-    // tiles of 64 keys) only for short contexts (measured on MI355X at
-    // D = 128: 4.7 against 7.5 us at 64 keys, 17.9 against 13.6 at 640).
-    if ((D == 64 || D == 128) && T <= 65535 && maxk <= ATT_DEC_MAXK) {
+    if (dec) {
         constexpr size_t LDS_MAX = 160 * 1024 - 64;
         const dim3 g((unsigned)(D / 32), (unsigned)H, (unsigned)T);
 #define ATT_DEC(F, DD)                                                                                           \

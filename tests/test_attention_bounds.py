@@ -284,7 +284,10 @@ def run_launch(T, H, Hkv, D, C, maxk, f16, kend, kstart, aligned=True):
     ranges = [att_range(kend, kstart, t, C, maxk) for t in range(T)]
     for k0, n in ranges:
         assert 0 <= k0 < C and 0 <= n <= min(C - k0, maxk)
-    G = H // Hkv
+    G, decw = H // Hkv, T * H * D // 32
+    if D in (64, 128) and maxk <= ATT_DEC_MAXK and (T < 16 or aligned and (decw <= 512 or decw <= 1024 and maxk <= 64)):
+        check_decode(b, ranges)
+        return "decode"
     if T >= 16 and D in (64, 128) and aligned:
         check_scores_mfma(b, ranges)
         each = b.kstart and G <= 4 and T * G * maxk <= 4 * C
@@ -295,9 +298,6 @@ def run_launch(T, H, Hkv, D, C, maxk, f16, kend, kstart, aligned=True):
         check_scores(b, ranges, 4)
         check_wsum_q4(b, ranges)
         return "many"
-    if D in (64, 128) and maxk <= ATT_DEC_MAXK:
-        check_decode(b, ranges)
-        return "decode"
     if D in (64, 128) and 2 <= G <= 8 and aligned and (maxk + 63) // 64 * Hkv * T >= 256:
         check_decode_scores(b, ranges)
         check_wsum(b, ranges)
@@ -350,7 +350,7 @@ def test_attention_addresses_in_bounds(D, f16):
 
 
 @pytest.mark.parametrize("T,H,Hkv,C,slots,maxk,path", [(37, 4, 4, 301, 1, 301, "mfma4"), (300, 32, 8, 301, 1, 301, "mfma16"),
-                                                      (37, 4, 4, 37 * 20, 37, 20, "each"), (8, 8, 2, 2047, 1, 2047, "two_grouped")])
+                                                      (37, 16, 16, 37 * 20, 37, 20, "each"), (8, 8, 2, 2047, 1, 2047, "two_grouped")])
 def test_missing_clamps_are_found(monkeypatch, T, H, Hkv, C, slots, maxk, path):
     """The checks of the matrix-core kernels fail when the restatement's
     clamps (rows past the last, keys and value blocks past the end) go."""
