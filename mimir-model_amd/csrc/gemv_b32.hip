@@ -15,8 +15,11 @@
 // checked against the oracle's restatement bit for bit and against the spec
 // tolerance.
 //
-// The chains are serial over K, the integer sums are not. A workgroup owns
-// eight weight rows and takes K in stages of 1024 elements in two phases:
+// Two forms, bit for bit the same.
+//
+// Two phases (gemv_b32_kernel), for grids that the latency of a chain's loads
+// would bound: the chains are serial over K, the integer sums are not. A
+// workgroup owns eight weight rows and takes K in stages of 1024 elements:
 // every thread multiplies 32 weights of one row with the M activation rows
 // (v_dot4_i32_i8, quants held in LDS) and leaves the eight sums as floats in
 // LDS; then a lane per (weight row, chain) of wave m % 4 runs the stage's
@@ -31,8 +34,14 @@
 // Q4_K 12.0 / 37.2 -> 8.8 / 19.1, Q6_K 35.5 / 130 -> 9.5 / 19.7; Q8_0
 // 14336 x 4096 at one row 35.5 -> 14.9 us, 2048 x 8192 57 -> 11.1 us.
 //
+// Direct (direct_kernel), where many weight rows keep the vector units busy by
+// themselves: a group of eight lanes per row, lane c running chain c in
+// registers, no sum through LDS. direct() below says which form runs.
+//
 // Rows of W with a non-finite block scale and refused activation rows take
 // the float32 path (reference interp/fast.go:323-377).
+#include <algorithm>
+
 #include "f32path.hpp"
 #include "kquant_lane.hpp"
 #include "mimg_device.hpp"
@@ -257,11 +266,131 @@ __global__ __launch_bounds__(256) void gemv_b32_kernel(Args A) {
     }
 }
 
+// Lane c of a group of eight owns elements 4c..4c+3 of every run of 32 of one
+// weight row, and with Q4_K the min of sub-block c; M activation rows.
+template <uint32_t DT, int M>
+__global__ __launch_bounds__(256) void direct_kernel(Args A) {
+    const int g = threadIdx.x >> 3, l = threadIdx.x & 7;
+    const int64_t row = (int64_t)blockIdx.x * 32 + g, rowc = min(row, A.N - 1);
+    const uint8_t* wrow = A.W + rowc * A.rb;
+    const int64_t K = A.K, R32 = K / 32, nb = DT == DT_Q8_0 ? R32 : K / 256;
+    float tot[M], off[M];
+#pragma unroll
+    for (int m = 0; m < M; m++) tot[m] = off[m] = 0.f;
+    for (int64_t b = 0; b < nb; b++) {
+        if constexpr (DT == DT_Q8_0) {
+            const uint8_t* blk = wrow + b * Q80_BYTES;
+            const uint32_t* a = (const uint32_t*)__builtin_align_down(blk + 2 + 4 * l, 4);
+            const uint32_t wq = __builtin_amdgcn_alignbyte(a[1], a[0], (uint32_t)((uintptr_t)(blk + 2) & 3));
+            const float dw = f16_to_f32(load_u16(blk));
+#pragma unroll
+            for (int m = 0; m < M; m++) {
+                const int P = sdot4(wq, *(const uint32_t*)(A.q + m * K + 32 * b + 4 * l), 0);
+                tot[m] = __builtin_fmaf((float)P, dw * A.d32[m * R32 + b], tot[m]);
+            }
+        } else if constexpr (DT == DT_Q4_K) {
+            const uint8_t* blk = wrow + b * Q4K_BYTES;
+            const u32x4 hdr = *(const u32x4a4*)blk;
+            const float d = f16_to_f32(hdr.x & 0xFFFFu), dmin = f16_to_f32(hdr.x >> 16);
+            const Q4KScales s = q4k_scales(hdr.y, hdr.z, hdr.w);
+            uint32_t qd[4];
+#pragma unroll
+            for (int c = 0; c < 4; c++) qd[c] = *(const uint32_t*)(blk + 16 + 32 * c + 4 * l);
+            const float dm = dmin * (float)byte_of(s.m, l);
+#pragma unroll
+            for (int m = 0; m < M; m++) {
+                const float* dx = A.d32 + m * R32 + 8 * b;
+                off[m] = __builtin_fmaf(dm, A.dbs[m * R32 + 8 * b + l], off[m]);
+                float a = 0.f, o = 0.f;
+#pragma unroll
+                for (int c = 0; c < 4; c++) {
+                    const int8_t* yc = A.q + m * K + 256 * b + 64 * c + 4 * l;
+                    const int lo = sdot4(qd[c] & 0x0F0F0F0Fu, *(const uint32_t*)yc, 0);
+                    const int hi = sdot4((qd[c] >> 4) & 0x0F0F0F0Fu, *(const uint32_t*)(yc + 32), 0);
+                    a = __builtin_fmaf((float)((int)byte_of(s.sc, 2 * c) * lo), dx[2 * c], a);
+                    o = __builtin_fmaf((float)((int)byte_of(s.sc, 2 * c + 1) * hi), dx[2 * c + 1], o);
+                }
+                tot[m] = __builtin_fmaf(d, a + o, tot[m]);
+            }
+        } else {
+            const uint8_t* blk = wrow + b * Q6K_BYTES;
+            const uint32_t sh = (uint32_t)((uintptr_t)blk & 3);  // 2-byte aligned blocks
+            auto load4 = [&](const uint8_t* p) {
+                const uint32_t* a = (const uint32_t*)__builtin_align_down(p, 4);
+                return __builtin_amdgcn_alignbyte(a[1], a[0], sh);
+            };
+            const float d = f16_to_f32(load_u16(blk + 208));
+            uint32_t ql[4], qh[2];
+#pragma unroll
+            for (int j = 0; j < 4; j++) ql[j] = load4(blk + 64 * (j >> 1) + 32 * (j & 1) + 4 * l);
+#pragma unroll
+            for (int h = 0; h < 2; h++) qh[h] = load4(blk + 128 + 32 * h + 4 * l);
+            int sc[8];
+#pragma unroll
+            for (int j = 0; j < 8; j++) sc[j] = (int)(int8_t)blk[192 + 8 * (j >> 2) + 2 * (j & 3) + (l >> 2)];
+#pragma unroll
+            for (int m = 0; m < M; m++) {
+                const float* dx = A.d32 + m * R32 + 8 * b;
+                float a = 0.f, o = 0.f;
+#pragma unroll
+                for (int j = 0; j < 8; j++) {
+                    const int h = j >> 2, p = j & 3;
+                    const uint32_t q6 = ((ql[2 * h + (p & 1)] >> (4 * (p >> 1))) & 0x0F0F0F0Fu) |
+                                        (((qh[h] >> (2 * p)) & 0x03030303u) << 4);
+                    const uint32_t yv = *(const uint32_t*)(A.q + m * K + 256 * b + 32 * j + 4 * l);
+                    const float v = (float)(sc[j] * (sdot4(q6, yv, 0) - 32 * sdot4(0x01010101u, yv, 0)));
+                    if (j % 2 == 0) a = __builtin_fmaf(v, dx[j], a);
+                    else o = __builtin_fmaf(v, dx[j], o);
+                }
+                tot[m] = __builtin_fmaf(d, a + o, tot[m]);
+            }
+        }
+    }
+    const bool wok = A.wref[rowc] == 0;
+#pragma unroll
+    for (int m = 0; m < M; m++) {
+        float r = DT == DT_Q4_K ? tot[m] - off[m] : tot[m];
+        r += __shfl_xor(r, 4);  // HSUM1, as above
+        r += __shfl_xor(r, 1);
+        r += __shfl_xor(r, 2);
+        if (!wok || !A.ok[m]) r = f32dot_g8<DT>(wrow, A.x + m * K, K, A.fused != 0);
+        if (A.bias) r += A.bias[rowc];
+        if (l == 0 && row < A.N) A.y[(int64_t)m * A.N + row] = r;
+    }
+}
+
+// The form for N x K weights and M activation rows: direct from the N on at
+// which it measured faster on MI355X (both forms timed with the quantizer at
+// every M, 13 N from 2048 to 128256 and 9 K from 256 to 8192). The two-phase
+// form's LDS traffic grows with N M; the direct form's cost is the latency of
+// its loads, which Q8_0's and Q6_K's 4-byte pieces of 2-byte aligned blocks
+// make long, so only a short K or many rows pay there. Time of the two-phase
+// form over the direct one's at M = 1 / 4 / 8:
+//   Q4_K  4096 x 4096 0.80 / 0.70 / 0.51, 11008 x 4096 0.98 / 0.94 / 1.24,
+//         14336 x 4096 0.98 / 1.04 / 1.46, 32768 x 2048 1.17 / 1.39 / 1.79,
+//         128256 x 2048 1.24 / 1.64 / 2.06, 8192 x 512 1.07 / 1.20 / 1.17
+//   Q8_0  14336 x 4096 0.44 / 0.58 / 0.79, 14336 x 1024 0.75 / 0.91 / 1.11,
+//         32768 x 2048 0.67 / 0.98 / 1.38, 128256 x 2048 0.52 / 0.86 / 1.50,
+//         32768 x 512 1.15 / 1.65 / 2.22
+//   Q6_K  32768 x 512 1.18 / 1.10 / 1.05, 22000 x 256 1.39 / 1.36 / 1.27,
+//         128256 x 1024 0.70 / 0.79 / 0.81
+static bool direct(uint32_t dt, int64_t N, int64_t K, int M) {
+    const bool part = K < 2048 && K % 1024 != 0;  // half a stage of the two-phase form is empty
+    if (dt == DT_Q4_K) return N >= (K < 512 ? 5000 : part ? 8192 : M >= 7 ? 9000 : M >= 5 ? 8192 : 12000);
+    if (dt == DT_Q6_K) return K < 512 ? N >= 12000 : K < 768 && N >= 32768;
+    if (M >= 7) return N >= std::min<int64_t>(std::max<int64_t>(12 * K, 6000), 22000);
+    if (M >= 5) return K <= 4096 && N >= std::min<int64_t>(std::max<int64_t>(18 * K, 8192), 32768);
+    if (M == 4) return K <= 1536 && N >= std::max<int64_t>(20 * K, 8192);
+    return K <= (M == 3 ? 768 : 512) && N >= 40 * K;
+}
+
 template <uint32_t DT, int M>
 static hipError_t launch(const Args& A, hipStream_t stream) {
-    const int64_t nwg = (A.N + R - 1) / R;
+    const bool dir = direct(DT, A.N, A.K, M);
+    const int64_t rows = dir ? 32 : R, nwg = (A.N + rows - 1) / rows;
     if (nwg > 0x7fffffff) return hipErrorInvalidValue;
-    hipLaunchKernelGGL((gemv_b32_kernel<DT, M>), dim3((unsigned)nwg), dim3(256), 0, stream, A);
+    if (dir) hipLaunchKernelGGL((direct_kernel<DT, M>), dim3((unsigned)nwg), dim3(256), 0, stream, A);
+    else hipLaunchKernelGGL((gemv_b32_kernel<DT, M>), dim3((unsigned)nwg), dim3(256), 0, stream, A);
     return hipGetLastError();
 }
 

@@ -65,3 +65,24 @@ def test_gemv_refusals(gpu, oracle, dt, rows):
         w[4, at:at + 2] = np.frombuffer(np.float16(np.inf).tobytes(), np.uint8)
 
     check(gpu, oracle, dt, 21, 1280, rows, seed=11, bias=True, edit=edit)
+
+
+# gemv_b32.hip's direct form: a group of eight lanes a weight row; on its line
+# and a row below it, rows that end inside a workgroup of 32
+@pytest.mark.parametrize("dt,n,k", [(Q4_K, 12000, 1024), (Q4_K, 11999, 1024), (Q4_K, 8193, 1536), (Q4_K, 5001, 256),
+                                    (Q6_K, 12001, 256), (Q6_K, 32769, 512), (Q8_0, 22001, 2048), (Q8_0, 20505, 96),
+                                    (Q8_0, 6143, 512), (Q8_0, 8200, 32)])
+@pytest.mark.parametrize("rows", [1, 2, 3, 4, 5, 6, 7, 8])
+def test_gemv_direct(gpu, oracle, dt, n, k, rows):
+    check(gpu, oracle, dt, n, k, rows, seed=rows + n, bias=rows % 2 == 0)
+
+
+@pytest.mark.parametrize("dt,n,k,rows", [(Q8_0, 8200, 1056, 7), (Q4_K, 12001, 1280, 3), (Q6_K, 12010, 256, 8)])
+def test_direct_refusals(gpu, oracle, dt, n, k, rows):
+    def edit(wb, x):
+        x[rows - 1, 7] = np.inf
+        w = wb.reshape(n, -1)
+        at = {Q4_K: 2, Q6_K: 208, Q8_0: 0}[dt]
+        w[[4, n - 1], at:at + 2] = np.frombuffer(np.float16(np.inf).tobytes(), np.uint8)
+
+    check(gpu, oracle, dt, n, k, rows, seed=11, bias=True, edit=edit)
