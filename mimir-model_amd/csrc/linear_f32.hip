@@ -292,7 +292,7 @@ static hipError_t launch_gemm(const DevWeight& w, const float* x, int64_t rows, 
     return launch_gemm_k<DT, WM, KS, false>(w, x, rows, bias, y, stream);
 }
 
-// ---- up to 8 activation rows -------------------------------------------------
+// ---- up to 8 activation rows, and chunks of them ------------------------------
 //
 // A lane per (weight row, chain): the 32 lanes of a half-wave are one row's
 // chains, with one accumulator per activation row. A workgroup owns 8 rows
@@ -315,8 +315,9 @@ __device__ __forceinline__ int2 unit_chain(int v) {
 
 template <uint32_t DT, int M, int PF>
 __global__ __launch_bounds__(256) void gemv_kernel(const uint8_t* __restrict__ W, int64_t rb, int64_t N, int64_t K,
-                                                   const float* __restrict__ x, const float* __restrict__ bias,
-                                                   float* __restrict__ y) {
+                                                   const float* __restrict__ x, int rows,
+                                                   const float* __restrict__ bias, float* __restrict__ y) {
+    const int m0 = blockIdx.y * M;  // activation rows m0 .. (past the last: the last again, unstored)
     __shared__ __align__(16) float lw[2][VR * VS];
     __shared__ __align__(16) float lx[2][M * 256];
     const int t = threadIdx.x, lane = t & 63;
@@ -336,7 +337,7 @@ __global__ __launch_bounds__(256) void gemv_kernel(const uint8_t* __restrict__ W
         w = vload<DT>(wrow, sc, v, K);
         const float* xp = x + min((int64_t)256 * sc + t, K - 1);
 #pragma unroll
-        for (int m = 0; m < M; m++) xv[m] = xp[(int64_t)m * K];
+        for (int m = 0; m < M; m++) xv[m] = xp[(int64_t)min(m0 + m, rows - 1) * K];
     };
     auto store = [&](int s, const VRaw& w, const float (&xv)[M]) {
         const int buf = s & 1;
@@ -392,35 +393,55 @@ __global__ __launch_bounds__(256) void gemv_kernel(const uint8_t* __restrict__ W
         r += __shfl_xor(r, 16);
         r += __shfl_xor(r, 4);
         r += __shfl_xor(r, 8);
-        if (n < N && (lane & 31) == 0) {
+        if (n < N && m0 + m < rows && (lane & 31) == 0) {
             if (bias) r += bias[n];
-            y[(int64_t)m * N + n] = r;
+            y[(int64_t)(m0 + m) * N + n] = r;
         }
     }
 }
 
 template <uint32_t DT, int M>
-static hipError_t launch_gemv(const DevWeight& w, const float* x, const float* bias, float* y, hipStream_t stream) {
+static hipError_t launch_gemv(const DevWeight& w, const float* x, int64_t rows, const float* bias, float* y,
+                              hipStream_t stream) {
     constexpr int PF = M <= 4 ? 4 : 3;
     const int64_t nwg = (w.n + VR - 1) / VR;
     if (nwg > 0x7fffffff) return hipErrorInvalidValue;
-    hipLaunchKernelGGL((gemv_kernel<DT, M, PF>), dim3((unsigned)nwg), dim3(256), 0, stream, w.data, w.row_bytes, w.n, w.k,
-                       x, bias, y);
+    hipLaunchKernelGGL((gemv_kernel<DT, M, PF>), dim3((unsigned)nwg, (unsigned)((rows + M - 1) / M)), dim3(256), 0, stream,
+                       w.data, w.row_bytes, w.n, w.k, x, (int)rows, bias, y);
     return hipGetLastError();
 }
 
 template <uint32_t DT>
 static hipError_t launch(const DevWeight& w, const float* x, int64_t rows, const float* bias, float* y,
                          hipStream_t stream) {
+    // The GEMV in chunks of activation rows where its grid is small: of one, two
+    // or four rows up to 256 workgroups (Q8_0 512; up to 8 rows only whole
+    // chunks), and for Q8_0, whose chains are the same above 8 rows, of eight
+    // rows up to 768. Measured on MI355X, us, in chunks / in one pass up to 8
+    // rows, in tiles above (10 N from 8 to 8192, 6 K): Q8_0 512 x 2048 at 8 rows
+    // 6.7 / 9.9, at 16 7.7 / 21.6, at 64 14.2 / 21.8, 2048 x 4096 at 16 rows
+    // 23.2 / 38; 1000 x 256 at 33 rows 6.3 / 7.3; in chunks of eight from 769 to
+    // 1024 workgroups at K <= 1024 0.96 to 1.07 of the tiles, up to 1536 1.29 to
+    // 1.53 at K <= 512; Q4_K 512 x 2048 at 8 rows 6.2 / 9.9.
+    if (rows <= 8 || DT == DT_Q8_0) {
+        const int64_t nwg = (w.n + VR - 1) / VR;
+        auto takes = [&](int m) {
+            return (rows > 8 || rows % m == 0) && nwg * ((rows + m - 1) / m) <= (DT == DT_Q8_0 ? 512 : 256);
+        };
+        if (takes(1)) return launch_gemv<DT, 1>(w, x, rows, bias, y, stream);
+        if (takes(2)) return launch_gemv<DT, 2>(w, x, rows, bias, y, stream);
+        if (takes(4)) return launch_gemv<DT, 4>(w, x, rows, bias, y, stream);
+        if (rows > 8 && nwg * ((rows + 7) / 8) <= 768) return launch_gemv<DT, 8>(w, x, rows, bias, y, stream);
+    }
     switch (rows) {
-    case 1: return launch_gemv<DT, 1>(w, x, bias, y, stream);
-    case 2: return launch_gemv<DT, 2>(w, x, bias, y, stream);
-    case 3: return launch_gemv<DT, 3>(w, x, bias, y, stream);
-    case 4: return launch_gemv<DT, 4>(w, x, bias, y, stream);
-    case 5: return launch_gemv<DT, 5>(w, x, bias, y, stream);
-    case 6: return launch_gemv<DT, 6>(w, x, bias, y, stream);
-    case 7: return launch_gemv<DT, 7>(w, x, bias, y, stream);
-    case 8: return launch_gemv<DT, 8>(w, x, bias, y, stream);
+    case 1: return launch_gemv<DT, 1>(w, x, rows, bias, y, stream);
+    case 2: return launch_gemv<DT, 2>(w, x, rows, bias, y, stream);
+    case 3: return launch_gemv<DT, 3>(w, x, rows, bias, y, stream);
+    case 4: return launch_gemv<DT, 4>(w, x, rows, bias, y, stream);
+    case 5: return launch_gemv<DT, 5>(w, x, rows, bias, y, stream);
+    case 6: return launch_gemv<DT, 6>(w, x, rows, bias, y, stream);
+    case 7: return launch_gemv<DT, 7>(w, x, rows, bias, y, stream);
+    case 8: return launch_gemv<DT, 8>(w, x, rows, bias, y, stream);
     }
     // Tiles of 32 x 64 where they give at least three quarters of the CUs a
     // workgroup, else 32 x 32, two workgroups a CU (measured on MI355X: 192

@@ -40,6 +40,23 @@ def test_rows_and_tiles(gpu, oracle, dt, k, rows, n):
     check(gpu, oracle, dt, n, k, rows, seed=rows + n, bias=rows % 2 == 1)
 
 
+# Q8_0 above 8 rows: chunks of the GEMV up to 768 workgroups of eight rows, a
+# last chunk of one to eight rows, and the tiles just past them
+@pytest.mark.parametrize("k", [32, 288, 1120, 1024])
+@pytest.mark.parametrize("rows,n", [(9, 3072), (9, 3080), (17, 2050), (33, 1297), (64, 768), (64, 801), (131, 401),
+                                    (10, 1100), (200, 33)])
+def test_q8_0_chunks_and_tiles(gpu, oracle, k, rows, n):
+    check(gpu, oracle, Q8_0, n, k, rows, seed=rows + n, bias=rows % 2 == 1)
+
+
+# up to 8 rows in chunks of one, two and four and in one pass
+@pytest.mark.parametrize("dt,k", [(Q4_K, 512), (Q6_K, 256), (Q8_0, 96)])
+@pytest.mark.parametrize("rows,n", [(2, 1024), (2, 1025), (4, 512), (4, 1030), (6, 600), (8, 250), (8, 300), (8, 1024), (8, 2056),
+                                    (7, 290), (7, 300), (8, 4100)])
+def test_gemv_chunks(gpu, oracle, dt, k, rows, n):
+    check(gpu, oracle, dt, n, k, rows, seed=rows + n, bias=rows % 4 == 0)
+
+
 @pytest.mark.parametrize("dt", [Q4_K, Q6_K, Q8_0])
 @pytest.mark.parametrize("rows", [3, 40])
 def test_non_finite(gpu, oracle, dt, rows):
@@ -83,7 +100,7 @@ def test_matrix_core_chain_is_fma(gpu, oracle, exponents):
     have the steps of calls of at most 8 (fmaf). Every value class of the
     activations, f16 scales of every finite class; a row with one NaN keeps
     its sign and payload (several NaNs: which one survives is the adds')."""
-    n, k, rows = 70, 1056, 40
+    n, k, rows = 1300, 1056, 40
     rng = np.random.default_rng(exponents[0] * 1000 + exponents[1])
     wb = rng.integers(0, 256, (n, k // 32, 34), dtype=np.uint8)
     d = rng.integers(0, 0x7C00, (n, k // 32), dtype=np.uint16) | rng.integers(0, 2, (n, k // 32), dtype=np.uint16) << 15
