@@ -325,16 +325,23 @@ static hipError_t launch(Args A, hipStream_t stream) {
 
 // 128 weight rows by 64 activation rows a workgroup where that gives more
 // than 256 workgroups, else by 32 rows where that gives at least 96; fewer:
-// not taken (the 16 x 16 x 64 tiles, gemm_kquant16.hip). Measured on MI355X,
+// not taken (the 16 x 16 x 64 tiles, gemm_kquant16.hip). Nor above 16 rows up to
+// 128 of them at one to three blocks a row, where the prologue weighs, if the other
+// tiles' grid is a full one. Measured on MI355X,
 // us with quantizing, 64-row tiles / 32-row tiles / 16 x 16 x 64 tiles:
 // 14336 x 4096 by 512 rows (896 workgroups of 64 rows) 89 / 95 / -, 4096 x
 // 4096 by 768 (384) 48.0 / 48.6, by 512 (256) 35.5 / 35.3, by 256 33 / 23.0 /
 // 25, by 96 (96 workgroups of 32 rows) - / 22.5 / 23.4, by 64 (64) - / 22.5 /
-// 19.5, 512 x 2048 by 181 (24) - / 14.7 / 14.9.
+// 19.5, 512 x 2048 by 181 (24) - / 14.7 / 14.9; 8192 x 512 by 48 (128) - / 9.9 /
+// 9.2, 4096 x 256 by 128 (128) - / 9.1 / 8.5, but 6144 x 512 by 64 (96; 192 of
+// the others) - / 9.9 / 12.8, 12288 x 512 by 64 (192) - / 10.3 / 10.9, 3072 x
+// 1024 by 181 (144) - / 12.2 / 13.3, 16384 x 512 by 16 (128) - / 8.8 / 9.3.
 bool launch_gemm_q4k(const DevWeight& w, const ActPtrs& a, int64_t rows, int64_t total_rows, const float* x,
                      const float* bias, float* y, hipStream_t stream, hipError_t* err) {
     const int64_t ntn = (w.n + 127) / 128;
-    if (ntn * ((rows + 31) / 32) < 96) return false;
+    const int64_t nwg = ntn * ((rows + 31) / 32);
+    if (nwg < 96) return false;
+    if (w.k < 1024 && rows > 16 && nwg <= 128 && (w.n + 31) / 32 * ((rows + 63) / 64) >= (rows <= 64 ? 256 : 192)) return false;
     gq4::Args A;
     A.W = w.data;
     A.wref = w.wref;

@@ -1,5 +1,5 @@
 """Q4_K prefill tiles (gemm_q4k.hip): 128 weight rows by 32 activation rows
-from 96 workgroups of those, by 64 above 256 workgroups; bit for bit the
+from 96 workgroups of those (129 at a short K and wide grids), by 64 above 256; bit for bit the
 oracle, at the edges of both tiles, on both sides of the rules, with bias and
 refusals (reference amx_test.go:41-141)."""
 import numpy as np
@@ -24,16 +24,18 @@ def check(gpu, oracle, rows, n, k, edit=None, bias=False):
     assert same.all(), f"{(~same).sum()} of {same.size} differ, first at {np.argwhere(~same)[0]}"
 
 
-# 95 and 96 tiles of 32 rows, 256 and 272 tiles of 64 rows, a lone last row of
-# a tile in each direction, one block and several
-@pytest.mark.parametrize("rows,n,k", [(31, 12160, 256), (31, 12161, 512), (32, 12289, 256), (97, 3073, 768),
-                                      (96, 4096, 1024), (1024, 2048, 256), (1025, 2048, 512), (65, 16513, 256),
+# 95 and 96 tiles of 32 rows at a longer K and, with few tiles of the other
+# kernel, at a short one, 128 and 130 at a short one, 256 and 272 tiles of 64 rows,
+# a lone last row of a tile in each direction, one block and several
+@pytest.mark.parametrize("rows,n,k", [(31, 12160, 1280), (31, 12161, 1280), (97, 3073, 1536), (64, 6144, 512),
+                                      (64, 6145, 256), (33, 8192, 512), (33, 8193, 512), (33, 12289, 256), (97, 6145, 768),
+                                      (192, 4096, 1024), (1024, 2048, 256), (1025, 2048, 512), (65, 16513, 256),
                                       (2047, 1025, 1024)])
 def test_tiles_and_rules(gpu, oracle, rows, n, k):
     check(gpu, oracle, rows, n, k, bias=rows % 2 == 1)
 
 
-@pytest.mark.parametrize("rows,n", [(100, 3100), (300, 7000)])
+@pytest.mark.parametrize("rows,n", [(250, 3100), (300, 7000)])
 def test_refusals(gpu, oracle, rows, n):
     def edit(wb, x):
         blocks = wb.reshape(n, 2, 144)
@@ -45,7 +47,7 @@ def test_refusals(gpu, oracle, rows, n):
     check(gpu, oracle, rows, n, 512, edit=edit, bias=True)
 
 
-@pytest.mark.parametrize("rows,n", [(100, 3100), (300, 7000)])
+@pytest.mark.parametrize("rows,n", [(250, 3100), (300, 7000)])
 def test_subnormal_scale_products(gpu, oracle, rows, n):
     """Scale products d * dx and dmin * dx that are subnormal, zero or among
     the smallest normal numbers: the outer product on the matrix cores rounds
