@@ -380,6 +380,62 @@ __global__ __launch_bounds__(256) void att_scores_kernel(const float* __restrict
     }
 }
 
+// Decode scores with grouped-query heads: a workgroup per (64 keys, kv
+// head, query) computes the scores of the G query heads that share the kv
+// head, each key loaded once for all G (att_scores_kernel loads it once per
+// query head). Every score's float steps are att_scores_kernel's (eight
+// lanes per key, lane c's fma chain over m, att_reduce8's pairing, times the
+// scale), so the results are bit for bit the same. The G heads' q rows are
+// loaded first (L2-resident), then the keys. Used where the launch rule
+// measures it ahead of the matrix cores' decode_scores_kernel: two heads leave
+// half of each matrix instruction idle, and the copy of 64 keys in LDS that a
+// wave there needs is twice as large in float32.
+template <bool F16, int DM, int G>
+__global__ __launch_bounds__(256) void att_scores_gqa_kernel(const float* __restrict__ q, const void* kc,
+                                                             const int64_t* __restrict__ kend,
+                                                             const int64_t* __restrict__ kstart, int T, int H, int Hkv,
+                                                             int D, int64_t C, int64_t maxk, float* __restrict__ ws) {
+    const int tile = blockIdx.x, hk = blockIdx.y, t = blockIdx.z;
+    const AttRange r = att_range(kend, kstart, t, C, maxk);
+    const int64_t n = r.n;
+    if ((int64_t)tile * 64 >= n) return;
+    const int lane = threadIdx.x & 63, c = lane & 7, gbase = lane & ~7, grp = threadIdx.x >> 3;
+    const float scale = (float)(1.0 / sqrt((double)D));
+    float qv[G][DM];
+#pragma unroll
+    for (int gi = 0; gi < G; gi++) {
+        const float* qr = q + ((int64_t)t * H + hk * G + gi) * D;
+#pragma unroll
+        for (int m = 0; m < DM; m++) qv[gi][m] = qr[8 * m + c];
+    }
+    const int64_t j0 = (int64_t)tile * 64 + grp, j1 = j0 + 32;
+    const int64_t base = (int64_t)hk * C + r.k0;
+    const int64_t a0 = base + (j0 < n ? j0 : n - 1), a1 = base + (j1 < n ? j1 : n - 1);  // past the end: the last key
+    float kv0[DM], kv1[DM];
+#pragma unroll
+    for (int m = 0; m < DM; m++) {
+        kv0[m] = kv_load<F16>(kc, a0 * D + 8 * m + c);
+        kv1[m] = kv_load<F16>(kc, a1 * D + 8 * m + c);
+    }
+    const int64_t n4 = n - n % 4;
+#pragma unroll
+    for (int gi = 0; gi < G; gi++) {
+        float l0 = 0.f, l1 = 0.f;
+#pragma unroll
+        for (int m = 0; m < DM; m++) {
+            l0 = __builtin_fmaf(qv[gi][m], kv0[m], l0);
+            l1 = __builtin_fmaf(qv[gi][m], kv1[m], l1);
+        }
+        const float p0 = att_reduce8(l0, j0 < n4, gbase, c);
+        const float p1 = att_reduce8(l1, j1 < n4, gbase, c);
+        float* out = ws + ((int64_t)t * H + hk * G + gi) * maxk;
+        if (c == 0) {
+            if (j0 < n) out[j0] = p0 * scale;
+            if (j1 < n) out[j1] = p1 * scale;
+        }
+    }
+}
+
 // One query's attention in one launch (decode): a workgroup per (DG dims,
 // head, query) computes all of the query's scores itself (the workgroups of
 // one head repeat them, each score in the same order), then the softmax and
@@ -1266,12 +1322,28 @@ hipError_t launch_attention(const float* q, const void* kc, const void* vc, cons
 #undef ATT_DEC
     }
     const int G = H / Hkv;
-    // the query heads of a kv head together (attention_mfma.hip), when that
-    // grid still gives every CU a wave (one query over a short context is
-    // faster per head: 4.1 against 4.5 us at 32 heads and 768 keys; from 512
-    // waves only, two queries of 2048 keys measured 22.0 for 20.0 us)
-    if ((D == 64 || D == 128) && G >= 2 && G <= 8 && (((uintptr_t)q | (uintptr_t)kc) & 15) == 0 &&
-        (long)tiles * Hkv * T >= 256) {
+    // the query heads of a kv head together, when that grid still gives every
+    // CU a workgroup or wave (one query over a short context is faster per
+    // head: 4.1 against 4.5 us at 32 heads and 768 keys; from 512 waves only,
+    // two queries of 2048 keys measured 22.0 for 20.0 us). On the matrix cores
+    // (attention_mfma.hip), except two heads a kv head, and four of a float32
+    // cache at D = 128, where the vector kernel is ahead. Whole call, matrix
+    // cores over vector kernel, median (largest) of the sizes from T = 1 to 15
+    // and 300 to 4096 keys: float32 G = 2 D = 64 1.01 (1.08), D = 128 1.04
+    // (1.10), G = 4 D = 128 1.02 (1.06); float16 G = 2 D = 128 1.02 (1.08)
+    // below 8192 waves and 0.98 above; G = 2 D = 64 0.99, G = 4 0.92 to 0.99,
+    // G = 8 0.89 to 0.99.
+    const long kvw = (long)tiles * Hkv * T;
+    if (kvw >= 256 && ((G == 2 && (f16 ? D == 128 && kvw < 8192 : D == 64 || D == 128)) || (G == 4 && !f16 && D == 128))) {
+        const dim3 grid(tiles, (unsigned)Hkv, (unsigned)T);
+#define ATT_GQA(F, DM, GG) \
+    hipLaunchKernelGGL((att_scores_gqa_kernel<F, DM, GG>), grid, dim3(256), 0, s, q, kc, kend, kstart, T, H, Hkv, D, C, maxk, ws)
+        if (f16) ATT_GQA(true, 16, 2);
+        else if (D == 64) ATT_GQA(false, 8, 2);
+        else if (G == 2) ATT_GQA(false, 16, 2);
+        else ATT_GQA(false, 16, 4);
+#undef ATT_GQA
+    } else if ((D == 64 || D == 128) && G >= 2 && G <= 8 && (((uintptr_t)q | (uintptr_t)kc) & 15) == 0 && kvw >= 256) {
         const hipError_t e = launch_att_scores_mfma(q, kc, kend, kstart, T, H, Hkv, D, C, maxk, f16, ws, s);
         if (e != hipSuccess) return e;
     } else {

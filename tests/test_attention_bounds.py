@@ -278,6 +278,20 @@ def check_decode_scores(b, ranges):
             assert n <= b.maxk
 
 
+def check_scores_gqa(b, ranges):
+    """att_scores_gqa_kernel: a workgroup per 64 keys, kv head and query."""
+    D, C, G = b.D, b.C, b.H // b.Hkv
+    for t, (k0, n) in enumerate(ranges):
+        for hk in {0, b.Hkv - 1}:
+            head0 = t * b.H + hk * G
+            b.check(head0 * D, (head0 + G) * D - 1, b.T * b.H * D, "scores_gqa: q")
+            for j0 in range(0, min(n, b.maxk), 64):
+                lo, hi = clamp(j0, n - 1), clamp(j0 + 63, n - 1)
+                b.check((hk * C + k0 + lo) * D, (hk * C + k0 + hi) * D + D - 1, (hk + 1) * C * D, "scores_gqa: key")
+                b.check(head0 * b.maxk + j0, (head0 + G - 1) * b.maxk + min(j0 + 63, n - 1), (head0 + G) * b.maxk,
+                        "scores_gqa: out")
+
+
 def run_launch(T, H, Hkv, D, C, maxk, f16, kend, kstart, aligned=True):
     b = Bounds(T, H, Hkv, D, C, maxk, f16)
     b.kstart = kstart is not None
@@ -298,7 +312,13 @@ def run_launch(T, H, Hkv, D, C, maxk, f16, kend, kstart, aligned=True):
         check_scores(b, ranges, 4)
         check_wsum_q4(b, ranges)
         return "many"
-    if D in (64, 128) and 2 <= G <= 8 and aligned and (maxk + 63) // 64 * Hkv * T >= 256:
+    kvw = (maxk + 63) // 64 * Hkv * T
+    if kvw >= 256 and (G == 2 and (f16 and D == 128 and kvw < 8192 or not f16 and D in (64, 128))
+                       or G == 4 and not f16 and D == 128):
+        check_scores_gqa(b, ranges)
+        check_wsum(b, ranges)
+        return "two_gqa"
+    if D in (64, 128) and 2 <= G <= 8 and aligned and kvw >= 256:
         check_decode_scores(b, ranges)
         check_wsum(b, ranges)
         return "two_grouped"
@@ -330,8 +350,10 @@ def test_attention_addresses_in_bounds(D, f16):
     rng = np.random.default_rng(D + (1000 if f16 else 0))
     seen = set()
     for T, (H, Hkv), C, slots, maxk_kind, aligned in itertools.product(
-            (1, 3, 8, 16, 37, 300), ((4, 1), (8, 2), (4, 4), (32, 8)), (1, 7, 42, 301, 2048, 8200), (1, 3, 40),
+            (1, 3, 8, 16, 37, 300), ((4, 1), (8, 2), (4, 4), (16, 8), (24, 8), (32, 8)), (1, 7, 42, 301, 2048, 8200), (1, 3, 40),
             ("C", "slot", "small", "max"), (True, False)):
+        if H in (16, 24) and (T != 8 or C != 2048 or D not in (64, 128)):
+            continue
         if slots > C or (H == 32 and T != 300) or (not aligned and (D not in (64, 128) or C > 301)):
             continue
         if (slots == 40) != (maxk_kind == "slot") or (slots == 40 and D not in (64, 128)):
@@ -342,7 +364,8 @@ def test_attention_addresses_in_bounds(D, f16):
         kend, kstart = ranges_for(T, C, maxk, slots, rng)
         seen.add(run_launch(T, H, Hkv, D, C, maxk, f16, kend, kstart if slots > 1 or T > 5 else None, aligned))
     if D in (64, 128):
-        assert seen == {"mfma4", "mfma16", "each", "many", "decode", "two", "two_grouped"}
+        gqa = set() if f16 and D == 64 else {"two_gqa"}
+        assert seen == {"mfma4", "mfma16", "each", "many", "decode", "two", "two_grouped"} | gqa
     elif D % 64 == 0:
         assert seen == {"many", "two"}
     else:

@@ -86,6 +86,16 @@ def test_decode_scores(gpu, oracle, f16, T, H, Hkv, D, C):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("f16", [False, True], ids=["f32cache", "f16cache"])
+@pytest.mark.parametrize("T,H,Hkv,D,C", [(3, 16, 8, 64, 705), (5, 8, 4, 128, 1290), (2, 32, 8, 128, 1023), (9, 64, 32, 128, 257),
+                                         (15, 4, 2, 64, 519)])
+def test_decode_scores_pairs(gpu, oracle, f16, T, H, Hkv, D, C):
+    """Two query heads a kv head, and four at D = 128: the vector kernel and
+    the matrix cores on either side of the line by cache type."""
+    test_decode_scores(gpu, oracle, f16, T, H, Hkv, D, C)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("f16", [False, True], ids=["f32cache", "f16cache"])
 @pytest.mark.parametrize("T,H,Hkv,D,slots,L", [(16, 4, 4, 64, 16, 261), (33, 6, 2, 128, 40, 83), (64, 8, 8, 128, 64, 29),
                                                (40, 8, 2, 64, 40, 300), (50, 4, 2, 128, 25, 131), (90, 3, 3, 64, 23, 71),
                                                (19, 1, 1, 128, 5, 700), (140, 2, 2, 128, 140, 7)])
