@@ -1,7 +1,7 @@
 #!/usr/bin/env python3
 """Benchmark of the block-quantized linear-layer path on one MI355X.
 
-Workload: the seven linear layers of one
+Workload (cfg1): the seven linear layers of one
 Llama-3-8B-shaped decoder layer at batch M = 1, Q4_K_M mixture
   q 4096->4096 Q4_K, k 4096->1024 Q4_K, v 4096->1024 Q6_K, o 4096->4096 Q4_K,
   gate/up 4096->14336 Q4_K, down 14336->4096 Q6_K,
@@ -39,10 +39,10 @@ weight bytes in one launch, timed the same way. The grouped gate+up launch
 (the roofline kernel of the grouped form), gate alone and the Q6_K down
 launch are reported beside it.
 
-cfg0 (BASELINE.json configs[0]): the single 4096 x 4096 Q4_K product of one
+cfg0: the single 4096 x 4096 Q4_K product of one
 activation row, quantized inside the launch, per call.
 
-prefill: the gate and down products at M = 64, 512, 2048
+prefill (cfg2): the gate and down products at M = 64, 512, 2048
 activation rows on the int8 matrix-core GEMMs (Q4_K/Q6_K with activation
 blocks of 256; Q8_0 with blocks of 32) and with float32 activations on the
 fp32 matrix cores. --prefill-only times only these and prints them as one
@@ -54,7 +54,7 @@ a bounded sample of the cfg1 layer set.
 
 The "decode" section runs whole greedy generation on the GPU decoder
 (mimir-model_amd/decoder.py) with random Q4_K_M weights of two model shapes
-(BASELINE.json configs[3] and [4]): a Llama-3.2-1B shape with a 32-token
+(cfg3 and cfg4): a Llama-3.2-1B shape with a 32-token
 prompt (uniform ids, seed 7) and 128 new tokens, and a Llama-3-8B shape
 with a 512-token prompt and 256 new tokens at batch 1 and at batch 8 (eight
 sequences in eight cache slots), f16 key-value cache. Reported: decode
@@ -146,7 +146,7 @@ def make_weights(stream, rotate, log):
 
 
 def make_q8_0_weights(stream, rotate, log):
-    """BASELINE configs[2]'s Q8_0 variant of gate (= up's shape) and down:
+    """cfg2's Q8_0 variant of gate (= up's shape) and down:
     the same f32 weights (seeds 4 and 6) encoded as Q8_0 (the reference's
     encoder, mim.Quantize), `rotate` device copies each."""
     layers = [dict() for _ in range(rotate)]
@@ -362,7 +362,7 @@ def main():
     args = ap.parse_args()
 
     if args.gpus != 1 or int(os.environ.get("WORLD_SIZE", "1")) != 1:
-        print("bench.py measures one GPU: this build has no multi-GPU path (row sharding is a design note). "
+        print("bench.py measures one GPU: libmimg has no multi-GPU path (row sharding is a design note). "
               "Run with --gpus 1.", file=sys.stderr)
         sys.exit(2)
 
@@ -381,12 +381,11 @@ def main():
     ws = [hiprt.DeviceBuffer(b) for b in ws_bytes]
     yd = {name: hiprt.DeviceBuffer(M * n * 4) for name, n, _, _, _, _ in CFG1}
 
-    # Prefill: the gate (Q4_K) and down (Q6_K) products
+    # Prefill (cfg2): the gate (Q4_K) and down (Q6_K) products
     # at M activation rows on the int8 MFMA GEMM, activations quantized
     # beforehand; a graph of --rotate launches over the rotation copies
     # (with --eager the same launches issued directly). Ops = 2*M*N*K; the fraction is of MI355X's dense int8 peak.
-    # With f32 (BASELINE.json north_star's f32-activation prefill,
-    # dequant_matmul.v1): the same products with float32 activations on the
+    # With f32 (f32-activation prefill, dequant_matmul.v1): the same products with float32 activations on the
     # fp32 matrix cores (mimg_linear_f32_mfma_dev), fraction of the dense
     # fp32 matrix peak.
     def prefill(name, rows, f32=False, q8_layers=None, b32=False):
@@ -726,7 +725,7 @@ def main():
         f"read+write); read kernel over 1 GiB {read_big_us[rb_per]:.1f} us "
         f"({hbm_ceiling['read_kernel_1GiB']['GB_per_s']:.0f} GB/s)")
 
-    # the single 4096 x 4096 Q4_K product (the q matrix,
+    # cfg0: the single 4096 x 4096 Q4_K product (the q matrix,
     # weight seed 0) of one activation row (seed 1), as the reference calls
     # it: dequant_matmul_a8.v2, x quantized inside the one-row launch; a
     # graph of --rotate calls over the rotation copies.

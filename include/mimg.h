@@ -237,7 +237,7 @@ int mimg_chain_status(void *sync, uint32_t *status);
  * mimg_linear_a8_set_workspace_bytes, 256-byte aligned), one launch runs all
  * the products, Q4_K and Q6_K mixed, so no product waits for another's
  * launch to drain. For a layer's linears whose inputs do not depend on each
- * other's outputs (BASELINE cfg1's linear set; a decoder layer's own calls
+ * other's outputs (cfg1 of the benchmark; a decoder layer's own calls
  * are dependent and keep mimg_linear_a8_group_dev). No output may overlap
  * any group's x or another output (MIMG_ERR_ARG). Returns MIMG_NOT_HANDLED
  * (nothing launched) unless every weight is Q4_K or Q6_K with K a multiple

@@ -1,7 +1,7 @@
-"""Writes cfg4_ids.json: the CPU restatement's greedy ids for BASELINE
-config 4 at its stated size, for tests/test_gpu_decoder.py.
+"""Writes cfg4_ids.json: the CPU restatement's greedy ids for the
+Llama-3-8B workload at its full size, for tests/test_gpu_decoder.py.
 
-Config 4's model is the Llama-3-8B shape (32 layers, d 4096, FFN 14336,
+The model is the Llama-3-8B shape (32 layers, d 4096, FFN 14336,
 32/8 heads, vocab 128256) with random Q4_K_M weights. The weights are drawn
 and encoded on the device (synthetic.build, seed 3, the same call the GPU
 tests make), so this script needs a GPU: it builds them, downloads their

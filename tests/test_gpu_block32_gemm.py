@@ -128,7 +128,7 @@ CFG2_Q8 = [("gate", 14336, 4096, 4), ("down", 4096, 14336, 6)]
 @pytest.mark.parametrize("rows", [64, 512, 2048])
 @pytest.mark.parametrize("name,n,k,seed", CFG2_Q8, ids=[c[0] for c in CFG2_Q8])
 def test_cfg2_q8_0_variant_within_a8_bound(gpu, oracle, name, n, k, seed, rows):
-    """BASELINE config 2's Q8_0 variant of gate/up and down at 64, 512 and
+    """The prefill workload's Q8_0 variant of gate/up and down at 64, 512 and
     2048 rows (62 MB of weights each): every output row of a spread sample
     of 64 rows within the bound (the float64 check of all rows would take
     minutes on the CPU)."""
@@ -306,7 +306,7 @@ CFG2_KQ = [("gate", Q4_K, 14336, 4096, 4), ("down", Q6_K, 4096, 14336, 6)]
 @pytest.mark.parametrize("rows", [64, 512])
 @pytest.mark.parametrize("name,dt,n,k,seed", CFG2_KQ, ids=[c[0] for c in CFG2_KQ])
 def test_cfg2_kquant_blocks_of_32_within_a8_bound(gpu, oracle, name, dt, n, k, seed, rows):
-    """BASELINE config 2's gate (Q4_K) and down (Q6_K) with activation
+    """The prefill workload's gate (Q4_K) and down (Q6_K) with activation
     blocks of 32 (a dequant_matmul_a8.v1 graph) at 64 and 512 rows: a spread
     sample of 64 output rows within the bound."""
     wb = oracle.synthetic_weight(dt, n, k, seed)

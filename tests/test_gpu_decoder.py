@@ -419,7 +419,7 @@ def _oracle_greedy(ref, prompt, n_new):
 
 @pytest.mark.parametrize("cache_f16", [False, True], ids=["f32cache", "f16cache"])
 def test_llama1b_shape_greedy_matches_oracle(gpu, cache_f16):
-    """the Llama-3.2-1B model shape (16 layers, d 2048,
+    """The Llama-3.2-1B model shape (16 layers, d 2048,
     FFN 8192, 32/8 heads, vocab 128256) with random Q4_K_M weights built on
     the device, a 32-token prompt (uniform ids, seed 7) and all 128 greedy
     tokens of the config; the GPU decoder and the CPU restatement, on the
@@ -442,7 +442,7 @@ def test_llama1b_shape_greedy_matches_oracle(gpu, cache_f16):
 
 @pytest.fixture(scope="module")
 def llama8b(gpu):
-    """BASELINE config 4's model: the Llama-3-8B shape (32 layers, d 4096,
+    """The Llama-3-8B shape (32 layers, d 4096,
     FFN 14336, 32/8 heads, vocab 128256) with random Q4_K_M weights drawn
     and encoded on the device (4.9 GB)."""
     import synthetic
@@ -1123,7 +1123,7 @@ def test_attention_many_queries_bitexact(gpu, oracle, rt, f16, T, slots, D, C):
 
 
 def test_container_upload_runs_match_the_go_executor(gpu):
-    """8(f)(3)/(4): the reference's importer output (a .mim container with
+    """The reference's importer output (a .mim container with
     its weights, metadata and graph) opened, its weights section uploaded in
     one transfer with every matrix a view at its offset, and the two runs of
     its compatibility fixture (a 7-token prompt, then one decode step at
@@ -1183,7 +1183,7 @@ def _release(g, sec, tensors, gpu):
 
 @pytest.mark.parametrize("name", fm.FIXTURES)
 def test_gguf_model_end_to_end(gpu, name):
-    """8(f)(4): the reference's GGUF fixture read by the product's GGUF
+    """The reference's GGUF fixture read by the product's GGUF
     reader, its tensor data uploaded in one transfer (views per matrix),
     the configuration from its metadata (LlamaConfigOf), and the reference's
     generate checks: f32 path within 2e-5 with the oracle's greedy ids; a8
@@ -1211,7 +1211,7 @@ def test_gguf_model_end_to_end(gpu, name):
 
 @pytest.mark.parametrize("name", fm.FIXTURES)
 def test_block32_a8_graph_matches_the_restatement(gpu, name):
-    """8(f)(4): dequant_matmul_a8.v1 (activation blocks of 32) for the Q4_K
+    """dequant_matmul_a8.v1 (activation blocks of 32) for the Q4_K
     and Q6_K matrices of the fixture model, the lane order of
     dotQ4KQ8AVX2/dotQ6KQ8AVX2: the GPU decoder's logits and greedy ids
     equal the CPU restatement's with the same block."""

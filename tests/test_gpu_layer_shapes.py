@@ -1,4 +1,4 @@
-"""BASELINE configs 0 and 2 at their full shapes, on the GPU through the C
+"""The single product and the prefill products at their full shapes, on the GPU through the C
 ABI, against the CPU oracle on the same bytes.
 
 cfg0 is the single 4096 x 4096 Q4_K product of one activation row (W from

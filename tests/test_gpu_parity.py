@@ -671,7 +671,7 @@ CFG1 = [  # (name, N, K, dtype, seed): Llama-3-8B layer, M = 1
 
 @pytest.mark.parametrize("name,n,k,dt,seed", CFG1)
 def test_cfg1_layer_shapes_bitexact(gpu, oracle, name, n, k, dt, seed):
-    """The BASELINE layer shapes at full size, M = 1 and M = 8: bit-exact."""
+    """The layer shapes at full size, M = 1 and M = 8: bit-exact."""
     wb = _weights(oracle, dt, n, k, seed)
     W = gpu.Weight(wb, dt, n, k)
     for rows in (1, 8):
