@@ -46,9 +46,11 @@
 // rows the chain of loads and reductions before the first product.
 // Measured on MI355X, us, against a key a lane for the scores and eight chains
 // a lane for the sum on the vector unit (32 heads, 8 kv heads, D = 128, f16):
-// 512 rows 125 -> 56 (scores 65 -> 24, sum 63 -> 32), 2000 rows 3197 -> 510,
-// 64 rows 37.7 -> 14.9, 16 rows 16.7 -> 13.9; D = 64: 512 rows 93 -> 62 (f16),
-// 94 -> 70 (f32). Loading the next tile's keys ahead in scores_kernel cost a
+// 512 rows 125 -> 53 (each kernel by itself: scores 65 -> 24, sum 63 -> 32),
+// 2000 rows 3197 -> 510, 64 rows 37.7 -> 14.9, 16 rows 16.7 -> 13.9; D = 64: 256
+// rows 51 -> 36, 512 rows 93 -> 62 (f16), 94 -> 70 (f32), 1000 rows 346 -> 130;
+// there, and with float32 values at D = 128, wsum's 16-row instances spill (33
+// registers for D = 64 f16, 73 f32, 11 for D = 128 f32). Loading the next tile's keys ahead in scores_kernel cost a
 // wave a SIMD and measured 61 us at 512 rows.
 #include <type_traits>
 
@@ -626,7 +628,9 @@ static hipError_t launch(const Args& A, hipStream_t s) {
     }
     hipLaunchKernelGGL((scores_kernel<F16, D, false>), g1, dim3(256), 0, s, A);
     // 16 rows a wave where that gives every CU a workgroup, else four (a
-    // quarter of the rows a workgroup, and a key of the chain in 6.9 ns, not 18)
+    // quarter of the rows a workgroup, and a key of the chain in 6.9 ns, not
+    // 18). The line was measured at D = 128 f16; at D = 64, whose 16-row
+    // instances spill, 181 rows of 32 heads (four) take 18 us and 256 (16) 36.
     const int64_t wt = (rows + 31) / 32 * A.Hkv;
     if (wt >= 256) hipLaunchKernelGGL((wsum_kernel<F16, D, 16, false>), dim3((unsigned)wt), dim3(2 * D), 0, s, A);
     else hipLaunchKernelGGL((wsum_kernel<F16, D, 4, false>), dim3((unsigned)((rows + 7) / 8 * A.Hkv)), dim3(2 * D), 0, s, A);

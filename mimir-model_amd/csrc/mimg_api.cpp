@@ -390,7 +390,7 @@ constexpr int64_t MFMA_MIN_ROWS = 4;
 // quantized into `a`; block-256 weights of one dtype share a launch per
 // chunk of 8 rows. Every path keeps each row's result independent of the
 // other rows of the call: block 256 from GEMM_MIN_ROWS on the MFMA GEMM
-// and blocks of 32 from GEMM_B32_MIN_ROWS on their own (Q8_0), each
+// and blocks of 32 from GEMM_B32_MIN_ROWS on their own (Q8_0 only), each
 // bit-identical to its GEMV, which takes the rest in chunks of eight.
 int matmul_quantized(const Weight* const* w, int count, const float* x, int64_t rows, const float* const* bias,
                      int block, float* const* y, const ActPtrs& a, hipStream_t s) {
